@@ -93,7 +93,9 @@ struct ArcW4A16Plan {
 // slices at once (slice_cols 64); kScheduleStream: one-row native plans on a persistent grid,
 // each workgroup streaming one contiguous range of slabs across slices with the whole activation
 // row staged in LDS (w4a16_gemv_stream.hip).
-enum Schedule : int { kScheduleRuns = 0, kSchedulePairs = 1, kScheduleStream = 2 };
+// kScheduleTiles: 17 rows and more on the row-tile GEMM (w4a16_gemm_tile.hip): m_tile x slice_cols
+// tiles, K in max_tile_contributors splits.
+enum Schedule : int { kScheduleRuns = 0, kSchedulePairs = 1, kScheduleStream = 2, kScheduleTiles = 3 };
 
 // The launch the GEMV will use for this shape on the current device. split_k_slices = 0 picks
 // the built-in policy; S > 0 gives every workgroup ceil(K / G / S) groups of whole 128-column

@@ -22,6 +22,7 @@
 #include <utility>
 
 #include "kernels/decode_quant_linear/w4a16_aux.h"
+#include "kernels/decode_quant_linear/w4a16_gemm_tile.h"
 #include "kernels/decode_quant_linear/w4a16_gemv.h"
 #include "ops/decode_quant_linear/w4a16_scratch.h"
 
@@ -150,6 +151,10 @@ constexpr int kMinRowsRunGroups = 16;
 constexpr int kMaxSlicesPerTile = 4;
 // Longest K for which one-row native plans stream slice pairs.
 constexpr int kMaxPairK = 4096;
+// Fewest rows the row-tile GEMM takes from the automatic dispatch: what the 2-16-row kernels, which
+// read the weights once for up to 16 rows, do not take (measured over 16 drawn shapes of 17-768
+// rows: 1.16-2.4 times faster than 16-row tiles).
+constexpr int kTileMinBatch = 17;
 
 // Grid, run length and fix-up workspace of a stream-K plan over tiles x slices x num_groups units.
 void finish_plan(ArcW4A16Plan& plan, long long tiles, long long slices, int num_groups,
@@ -222,6 +227,8 @@ bool arc_quarter_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_siz
                       int split_k_slices, int cu_count, bool cu_count_given);
 bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size,
                           int split_k_slices, int cu_count, bool cu_count_given);
+bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool silu,
+               int cu_count);
 
 }  // namespace
 
@@ -230,6 +237,10 @@ ArcW4A16Plan plan_arc_w4a16_for_cu_count(int batch, int n, int k, int group_size
   validate_dimensions(batch, n, k, group_size);
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, fk::gemv_m_tile_for_batch(batch));
+  if (split_k_slices == 0 && batch >= kTileMinBatch &&
+      tile_plan(plan, batch, n, k, group_size, false, cu_count)) {
+    return plan;
+  }
   if (!arc_mfma_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true) &&
       !arc_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true)) {
     arc_quarter_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true);
@@ -751,10 +762,36 @@ bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group
          mfma_stream_plan(plan, batch, n, k, group_size, true, cu_count, cu_count_given);
 }
 
+// The row-tile GEMM (w4a16_gemm_tile.hip). More than kTileMaxRows rows run as several launches over
+// one workspace. False (plan unchanged) when the tiles outnumber the fix-up counters.
+bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool silu,
+               int cu_count) {
+  const int rows = std::min(batch, fk::kTileMaxRows);
+  const fk::TileShape s =
+      fk::tile_shape(rows, n, k, group_size, silu, cu_count, kCounterRegionBytes);
+  std::size_t bytes = s.end;
+  if (const int rest = batch % fk::kTileMaxRows; rest != 0 && rest != rows) {
+    bytes = std::max(
+        bytes, fk::tile_shape(rest, n, k, group_size, silu, cu_count, kCounterRegionBytes).end);
+  }
+  if (static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters) {
+    return false;
+  }
+  plan = ArcW4A16Plan{};
+  plan.m_tile = s.bm;
+  plan.schedule = kScheduleTiles;
+  plan.slice_cols = s.bn;
+  plan.workgroups = s.grid;
+  plan.groups_per_workgroup = s.per * s.unit_groups;
+  plan.max_tile_contributors = s.splits;
+  plan.workspace_bytes = bytes;
+  return true;
+}
+
 // plan_w4a16_for_format for a kernel choice (kKernelDot2 is what the fused kernels need).
 ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int activation_dtype,
                                   int split_k_slices, int cu_count, int packet_format,
-                                  int kernel, bool plain = true) {
+                                  int kernel, bool plain = true, bool tiles = true) {
   const fk::PacketFormat format = to_packet_format(packet_format, true);
   validate_dimensions(batch, n, k, group_size);
   const bool cu_count_given = cu_count > 0;
@@ -763,6 +800,10 @@ ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int a
   }
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, m_tile_for_kernel(batch, kernel));
+  if (plain && tiles && split_k_slices == 0 && batch >= kTileMinBatch && kernel == kKernelAuto &&
+      tile_plan(plan, batch, n, k, group_size, false, cu_count)) {
+    return plan;
+  }
   if (plain && split_k_slices == 0 && batch >= kMfmaStreamMinBatch &&
       batch <= kMfmaStreamMaxBatch && kernel != kKernelDot2 && mfma_stream_enabled() &&
       (format != fk::PacketFormat::kArc || arc_mfma_stream_enabled()) &&
@@ -961,13 +1002,40 @@ struct StreamWorkspace {
   std::size_t bytes = 0;
 };
 
-void* library_workspace(std::size_t bytes, hipStream_t stream) {
-  static std::map<std::pair<int, hipStream_t>, StreamWorkspace> spaces;
-  static std::mutex mutex;
+struct StreamWorkspaces {
+  std::map<std::pair<int, hipStream_t>, StreamWorkspace> spaces;
+  std::mutex mutex;
+};
+
+StreamWorkspaces& stream_workspaces() {
+  static StreamWorkspaces all;
+  return all;
+}
+
+// Whether library_workspace(bytes, stream) can be had now: it is large enough already, or the
+// stream is not being captured.
+bool library_workspace_ready(std::size_t bytes, hipStream_t stream) {
   int device = 0;
   check_hip(hipGetDevice(&device), "hipGetDevice");
-  std::lock_guard<std::mutex> lock(mutex);
-  StreamWorkspace& ws = spaces[{device, stream}];
+  {
+    StreamWorkspaces& all = stream_workspaces();
+    std::lock_guard<std::mutex> lock(all.mutex);
+    const auto it = all.spaces.find({device, stream});
+    if (it != all.spaces.end() && it->second.bytes >= bytes) {
+      return true;
+    }
+  }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  check_hip(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
+  return status == hipStreamCaptureStatusNone;
+}
+
+void* library_workspace(std::size_t bytes, hipStream_t stream) {
+  int device = 0;
+  check_hip(hipGetDevice(&device), "hipGetDevice");
+  StreamWorkspaces& all = stream_workspaces();
+  std::lock_guard<std::mutex> lock(all.mutex);
+  StreamWorkspace& ws = all.spaces[{device, stream}];
   if (ws.bytes < bytes) {
     if (ws.ptr != nullptr) {
       check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
@@ -1076,6 +1144,34 @@ void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::u
     l.partials = static_cast<char*>(workspace) + kCounterRegionBytes;
   }
   check_hip(fk::launch_w4a16_gemv(l, stream), "w4a16_gemv launch");
+}
+
+// The launches of a kScheduleTiles plan.
+void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
+               std::uintptr_t output_ptr, void* workspace, int batch, int n, int k, int group_size,
+               int activation_dtype, hipStream_t stream, fk::PacketFormat format, bool silu = false,
+               std::uintptr_t norm_weight_ptr = 0, float eps = 0.0f) {
+  const int cu_count = device_cu_count();
+  for (int row = 0; row < batch; row += fk::kTileMaxRows) {
+    fk::TileLaunch l;
+    l.M = std::min(batch - row, fk::kTileMaxRows);
+    l.N = n;
+    l.K = k;
+    l.group_size = group_size;
+    l.act = activation_dtype == kActivationBF16 ? fk::Act::kBF16 : fk::Act::kF16;
+    l.format = format;
+    l.x = reinterpret_cast<const void*>(activations_ptr + static_cast<std::size_t>(row) * k * 2);
+    l.packets = reinterpret_cast<const void*>(packets_ptr);
+    l.out = reinterpret_cast<void*>(output_ptr +
+                                    static_cast<std::size_t>(row) * (silu ? n / 2 : n) * 2);
+    l.workspace = workspace;
+    l.silu = silu;
+    l.norm_weight = reinterpret_cast<const void*>(norm_weight_ptr);
+    l.eps = eps;
+    const fk::TileShape s =
+        fk::tile_shape(l.M, n, k, group_size, silu, cu_count, kCounterRegionBytes);
+    check_hip(fk::launch_w4a16_gemm_tile(l, s, stream), "w4a16_gemm_tile launch");
+  }
 }
 
 void validate_forward_buffers(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
@@ -1211,9 +1307,20 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
   validate_packet_stride(group_size, packet_stride_bytes);
   validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  const ArcW4A16Plan plan =
+  ArcW4A16Plan plan =
       plan_arc_w4a16_for_cu_count(batch, n, k, group_size, kActivationF16, 0, device_cu_count());
+  if (plan.schedule == kScheduleTiles && !library_workspace_ready(plan.workspace_bytes, stream)) {
+    // A captured call cannot allocate: the per-tile kernels need no prepared activations (and no
+    // workspace at all for most shapes).
+    plan = plan_for_format_impl(batch, n, k, group_size, kActivationF16, 0, device_cu_count(),
+                                kPacketArc, kKernelAuto, /*plain=*/true, /*tiles=*/false);
+  }
   void* workspace = plan.workspace_bytes > 0 ? library_workspace(plan.workspace_bytes, stream) : nullptr;
+  if (plan.schedule == kScheduleTiles) {
+    run_tiles(activations_ptr, packets_ptr, output_ptr, workspace, batch, n, k, group_size,
+              kActivationF16, stream, fk::PacketFormat::kArc);
+    return;
+  }
   run_gemv(activations_ptr, packets_ptr, output_ptr, workspace, plan, batch, n, k, group_size,
            kActivationF16, stream);
 }
@@ -1370,6 +1477,12 @@ void forward_with_format(std::uintptr_t activations_ptr, std::uintptr_t packets_
       throw_invalid(oss.str());
     }
   }
+  if (plan.schedule == kScheduleTiles) {
+    run_tiles(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr),
+              batch, n, k, group_size, activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr),
+              format);
+    return;
+  }
   run_gemv(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr), plan,
            batch, n, k, group_size, activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr),
            format);
@@ -1503,8 +1616,9 @@ void w4a16_forward_noalloc(std::uintptr_t activations_ptr, std::uintptr_t packet
   // The plan of arc_w4a16_forward_native, checked against the scratch size before any device
   // work; then the set-up on the first call on a device (address lookup, counter clear), and the
   // launch with the scratch array standing in for the workspace.
-  const ArcW4A16Plan plan = plan_w4a16_for_kernel(batch, n, k, group_size, activation_dtype, 0,
-                                                  device_cu_count(), packet_format, kKernelAuto);
+  const ArcW4A16Plan plan =
+      plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, device_cu_count(),
+                           packet_format, kKernelAuto, /*plain=*/true, /*tiles=*/false);
   if (plan.workspace_bytes > kNoAllocScratchBytes) {
     std::ostringstream oss;
     oss << "this launch needs " << plan.workspace_bytes << " bytes of fix-up scratch; the "

@@ -48,6 +48,9 @@ _IMPL_KERNEL = {_ARC_IMPL_AUTO: KERNEL_AUTO, _ARC_IMPL_SCALAR: KERNEL_DOT2,
                 _ARC_IMPL_MFMA: KERNEL_MFMA}
 _VENDOR_WORKSPACE_BYTES = 32 * 1024 * 1024
 
+# Plan schedule of the row-tile GEMM (FK_SCHEDULE_TILES in include/fk_w4a16.h)
+SCHEDULE_TILES = 3
+
 ACT_F16 = 0
 ACT_BF16 = 1
 
@@ -207,6 +210,20 @@ def arc_workspace(device: Any, nbytes: int) -> Any:
         ws = torch.zeros(size, device=device, dtype=torch.uint8)
         _ARC_WORKSPACE_CACHE[key] = ws
     return ws
+
+
+def _plan_workspace(plan: dict[str, int], device: Any) -> tuple[Any, int, int]:
+    """(tensor to keep until the launch, pointer, bytes) of a plan's workspace. A row-tile plan's
+    (prepared activations, partial tiles) grows with the rows and needs no zeros: it is the
+    allocator's, for this call. The others' counters are kept per stream (arc_workspace)."""
+    nbytes = int(plan["workspace_bytes"])
+    if nbytes == 0:
+        return None, 0, 0
+    if plan["schedule"] == SCHEDULE_TILES:
+        ws = _require_torch().empty(nbytes, device=device, dtype=_require_torch().uint8)
+    else:
+        ws = arc_workspace(device, nbytes)
+    return ws, ws.data_ptr(), ws.numel()
 
 
 def _split_k_partials(*, device: Any, batch: int, n: int, split_k_slices: int) -> Any:
@@ -428,12 +445,7 @@ def arc_w4a16_forward(
     requested = 0 if split_k_slices is None else split_k_slices
     kernel = _IMPL_KERNEL[resolved]
     plan = native.arc_w4a16_plan(batch, n, k, group_size, act, requested, 0, 0, kernel)
-    ws_bytes = int(plan["workspace_bytes"])
-    ws_ptr = 0
-    if ws_bytes > 0:
-        ws = arc_workspace(activations.device, ws_bytes)
-        ws_ptr = ws.data_ptr()
-        ws_bytes = ws.numel()
+    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
     if kernel != KERNEL_AUTO:
         native.w4a16_forward_kernel(
             activations.data_ptr(), packets.data_ptr(), output.data_ptr(), ws_ptr, ws_bytes,

@@ -35,8 +35,8 @@ from fast_kernels.ops.decode_quant_linear import (
     _current_stream_ptr,
     _require_gpu_backend,
     _require_torch,
+    _plan_workspace,
     arc_packet_stride_bytes,
-    arc_workspace,
 )
 
 if TYPE_CHECKING:  # pragma: no cover
@@ -238,10 +238,7 @@ def arc_w4a16_forward_native(
     requested = 0 if split_k_slices is None else int(split_k_slices)
     act = _act_code(activations.dtype)
     plan = native.arc_w4a16_plan(batch, n, k, group_size, act, requested, 0, code)
-    ws_ptr, ws_bytes = 0, int(plan["workspace_bytes"])
-    if ws_bytes > 0:
-        ws = arc_workspace(activations.device, ws_bytes)
-        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
     native.arc_w4a16_forward_native(
         activations.data_ptr(), packets.data_ptr(), output.data_ptr(), ws_ptr, ws_bytes, batch,
         n, k, group_size, code, act, requested, _current_stream_ptr(activations.device),
@@ -293,10 +290,7 @@ def arc_w4a16_forward_rmsnorm(
     requested = 0 if split_k_slices is None else int(split_k_slices)
     act = _act_code(activations.dtype)
     plan = native.w4a16_plan_rmsnorm(batch, n, k, group_size, act, requested, 0, code)
-    ws_ptr, ws_bytes = 0, int(plan["workspace_bytes"])
-    if ws_bytes > 0:
-        ws = arc_workspace(activations.device, ws_bytes)
-        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
     native.w4a16_forward_rmsnorm(
         activations.data_ptr(), norm_weight.data_ptr(), float(eps), packets.data_ptr(),
         output.data_ptr(), ws_ptr, ws_bytes, batch, n, k, group_size, code, act, requested,
