@@ -48,6 +48,18 @@ void call(Fn&& fn) {
   check(status);
 }
 
+py::dict plan_dict(const fk_arc_w4a16_plan& plan) {
+  py::dict d;
+  d["m_tile"] = plan.m_tile;
+  d["workgroups"] = plan.workgroups;
+  d["groups_per_workgroup"] = plan.groups_per_workgroup;
+  d["max_tile_contributors"] = plan.max_tile_contributors;
+  d["workspace_bytes"] = plan.workspace_bytes;
+  d["slice_cols"] = plan.slice_cols;
+  d["schedule"] = plan.schedule;
+  return d;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
@@ -212,15 +224,7 @@ PYBIND11_MODULE(_native, m) {
         fk_arc_w4a16_plan plan{};
         check(fk_w4a16_plan_for_kernel(batch, n, k, group_size, activation_dtype, split_k_slices,
                                        cu_count, packet_format, kernel, &plan));
-        py::dict d;
-        d["m_tile"] = plan.m_tile;
-        d["workgroups"] = plan.workgroups;
-        d["groups_per_workgroup"] = plan.groups_per_workgroup;
-        d["max_tile_contributors"] = plan.max_tile_contributors;
-        d["workspace_bytes"] = plan.workspace_bytes;
-        d["slice_cols"] = plan.slice_cols;
-        d["schedule"] = plan.schedule;
-        return d;
+        return plan_dict(plan);
       },
       py::arg("batch"), py::arg("n"), py::arg("k"), py::arg("group_size"),
       py::arg("activation_dtype") = FK_ACT_F16, py::arg("split_k_slices") = 0,
@@ -333,15 +337,7 @@ PYBIND11_MODULE(_native, m) {
         fk_arc_w4a16_plan plan{};
         check(fk_w4a16_plan_rmsnorm(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, packet_format, &plan));
-        py::dict d;
-        d["m_tile"] = plan.m_tile;
-        d["workgroups"] = plan.workgroups;
-        d["groups_per_workgroup"] = plan.groups_per_workgroup;
-        d["max_tile_contributors"] = plan.max_tile_contributors;
-        d["workspace_bytes"] = plan.workspace_bytes;
-        d["slice_cols"] = plan.slice_cols;
-        d["schedule"] = plan.schedule;
-        return d;
+        return plan_dict(plan);
       },
       py::arg("batch"), py::arg("n"), py::arg("k"), py::arg("group_size"),
       py::arg("activation_dtype"), py::arg("split_k_slices"), py::arg("cu_count"),
@@ -380,4 +376,34 @@ PYBIND11_MODULE(_native, m) {
       py::arg("n"), py::arg("k"), py::arg("group_size"), py::arg("packet_format"),
       py::arg("activation_dtype"), py::arg("norm_weight_ptr"), py::arg("eps"),
       py::arg("stream_ptr"));
+  m.def(
+      "w4a16_plan_fused",
+      [](int batch, int n, int k, int group_size, int activation_dtype, int cu_count,
+         int packet_format, bool silu) {
+        fk_arc_w4a16_plan plan{};
+        check(fk_w4a16_plan_fused(batch, n, k, group_size, activation_dtype, cu_count,
+                                  packet_format, silu, &plan));
+        return plan_dict(plan);
+      },
+      py::arg("batch"), py::arg("n"), py::arg("k"), py::arg("group_size"),
+      py::arg("activation_dtype"), py::arg("cu_count"), py::arg("packet_format"),
+      py::arg("silu"));
+  m.def(
+      "w4a16_forward_fused",
+      [](std::uintptr_t activations_ptr, std::uintptr_t norm_weight_ptr, float eps,
+         std::uintptr_t packets_ptr, std::uintptr_t output_ptr, std::uintptr_t workspace_ptr,
+         std::size_t workspace_bytes, int batch, int n, int k, int group_size, int packet_format,
+         int activation_dtype, bool silu, std::uintptr_t stream_ptr) {
+        call([&] {
+          return fk_w4a16_forward_fused(cp(activations_ptr), cp(norm_weight_ptr), eps,
+                                        cp(packets_ptr), mp(output_ptr), mp(workspace_ptr),
+                                        workspace_bytes, batch, n, k, group_size, packet_format,
+                                        activation_dtype, silu, mp(stream_ptr));
+        });
+      },
+      py::arg("activations_ptr"), py::arg("norm_weight_ptr"), py::arg("eps"),
+      py::arg("packets_ptr"), py::arg("output_ptr"), py::arg("workspace_ptr"),
+      py::arg("workspace_bytes"), py::arg("batch"), py::arg("n"), py::arg("k"),
+      py::arg("group_size"), py::arg("packet_format"), py::arg("activation_dtype"),
+      py::arg("silu"), py::arg("stream_ptr"));
 }

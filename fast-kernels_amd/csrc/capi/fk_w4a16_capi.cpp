@@ -300,4 +300,27 @@ int fk_w4a16_forward_silu_mul(const void* activations, const void* packets, void
   });
 }
 
+int fk_w4a16_plan_fused(int batch, int n, int k, int group_size, int activation_dtype,
+                        int cu_count, int packet_format, int silu, fk_arc_w4a16_plan* plan) {
+  return guarded([&] {
+    if (plan == nullptr) {
+      throw std::invalid_argument("plan must not be null");
+    }
+    copy_plan(ops::plan_w4a16_fused(batch, n, k, group_size, activation_dtype, cu_count,
+                                    packet_format, silu != 0),
+              plan);
+  });
+}
+
+int fk_w4a16_forward_fused(const void* activations, const void* norm_weight, float eps,
+                           const void* packets, void* output, void* workspace,
+                           size_t workspace_bytes, int batch, int n, int k, int group_size,
+                           int packet_format, int activation_dtype, int silu, void* stream) {
+  return guarded([&] {
+    ops::w4a16_forward_fused(P(activations), P(norm_weight), eps, P(packets), P(output),
+                             P(workspace), workspace_bytes, batch, n, k, group_size, packet_format,
+                             activation_dtype, silu != 0, P(stream));
+  });
+}
+
 }  // extern "C"

@@ -340,4 +340,36 @@ int fk_w4a16_forward_silu_mul(const void* activations, const void* packets, void
   return FK_ERR_RUNTIME;
 }
 
+int fk_w4a16_plan_fused(int batch, int n, int k, int group_size, int activation_dtype, int cu_count, int packet_format, int silu, fk_arc_w4a16_plan* plan) {
+  (void)batch;
+  (void)n;
+  (void)k;
+  (void)group_size;
+  (void)activation_dtype;
+  (void)cu_count;
+  (void)packet_format;
+  (void)silu;
+  (void)plan;
+  return FK_ERR_RUNTIME;
+}
+
+int fk_w4a16_forward_fused(const void* activations, const void* norm_weight, float eps, const void* packets, void* output, void* workspace, size_t workspace_bytes, int batch, int n, int k, int group_size, int packet_format, int activation_dtype, int silu, void* stream) {
+  (void)activations;
+  (void)norm_weight;
+  (void)eps;
+  (void)packets;
+  (void)output;
+  (void)workspace;
+  (void)workspace_bytes;
+  (void)batch;
+  (void)n;
+  (void)k;
+  (void)group_size;
+  (void)packet_format;
+  (void)activation_dtype;
+  (void)silu;
+  (void)stream;
+  return FK_ERR_RUNTIME;
+}
+
 }  // extern "C"

@@ -30,6 +30,7 @@
 //    for window j, the 8 bytes of columns 32 q + 2 n and + 1 in word row 4 j + t (four 128-byte
 //    runs per load) and those columns' alphas and betas; the two chains are the two columns, A
 //    the staged k-chunk 4 j + t, and the epilogue y += alpha D + beta S with the packet's betas.
+//  * kFuse: the RMSNorm prologue and the SiLU epilogue of a decode step (see the kernel).
 //  * kParts (rows too long to stage whole): K in stream_parts equal parts; workgroup b takes part
 //    b / (grid / parts) of its whole slices, stages only that part's activations, and writes its
 //    fp32 partial tiles to partials [parts, M, N]; add_parts_kernel then adds the parts in part
@@ -127,10 +128,18 @@ __device__ __forceinline__ void arc_mfma_load(ArcMfmaLoad<G>& ld, const uint8_t*
 // host keeps launches within it.
 constexpr int max_stage_per_lane(int mt) { return mt; }
 
-template <int G, Act A, PacketFormat F, int kW, int D, int MT, bool kPieces, bool kParts = false>
+// kFuse (native slabs, whole slices): the RMSNorm prologue, whose row sums come from the staging's
+// own loads (every workgroup stages whole rows) at the cost of one barrier, and the SiLU epilogue,
+// for which a workgroup streams its gate slices and then the same up slices.
+template <int G, Act A, PacketFormat F, int kW, int D, int MT, bool kPieces, bool kParts = false,
+          GemvFuse kFuse = GemvFuse::kNone>
 __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
     w4a16_gemm_mfma_stream_kernel(GemvParams p) {
   static_assert(!(kPieces && kParts), "pieces or K parts, not both");
+  constexpr bool kNorm = kFuse == GemvFuse::kRmsNorm || kFuse == GemvFuse::kRmsNormSiluMul;
+  constexpr bool kSilu = kFuse == GemvFuse::kSiluMul || kFuse == GemvFuse::kRmsNormSiluMul;
+  static_assert(kFuse == GemvFuse::kNone || (is_native(F) && !kPieces && !kParts),
+                "fused neighbours on whole slices of native slabs");
   extern __shared__ uint4 mfma_stream_lds[];
   constexpr int WR = G / 8;
   constexpr int U = native_unit_words(G);
@@ -164,7 +173,12 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
   const int slices = p.N / kSliceCols;
   const int rows = p.M;  // rows < MT are real, the rest zeros
   const int n_out = rows * kSliceCols;
-  const StreamRange rg = stream_range(b, grid, p.stream_whole, slices, nbs, kPieces);
+  StreamRange rg = stream_range(b, grid, p.stream_whole, slices, nbs, kPieces);
+  // kSilu: the workgroup's gate slices from slice b * pairs on, then the same up slices
+  const int pairs = kSilu ? p.stream_whole / 2 : 0;
+  if constexpr (kSilu) {
+    rg.whole_slice0 = b * pairs;
+  }
   constexpr bool kArcPk = F == PacketFormat::kArc;
   using Load = std::conditional_t<kArcPk, ArcMfmaLoad<G>, NativeLoad<G>>;
 
@@ -227,9 +241,14 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
   const int off_w = rg.whole_slice0 * ng + wave - (n_h + n_t) * kW;
   const int off_t = rg.tail_slice * ng + wave - n_h * kW;
   const int off_h = rg.head_slice * ng + rg.head_blk0 * Q + wave;
+  const int n_gate = pairs * nbs * D;                // the wave's gate slabs (kSilu)
+  const int up_jump = (slices / 2 - pairs) * ng;     // slabs from the last gate slice to the up ones
   auto slab = [&](int i) __attribute__((always_inline)) -> const uint8_t* {
     const int c = min(i, j_last);
     int off = off_w;
+    if constexpr (kSilu) {
+      off += __builtin_amdgcn_readfirstlane(c >= n_gate ? 1 : 0) * up_jump;
+    }
     if constexpr (kPieces) {
       // 0/1 flags made opaque to the compiler (readfirstlane), which otherwise turns the choice
       // into a lookup table in scratch memory
@@ -312,6 +331,17 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
     const int m = min(pass_row(i), rows - 1);  // rows past the batch: read a real row, stage 0
     raw[i] = *reinterpret_cast<const uint4*>(p.x + (m * p.K + (g0 + g) * G + wr * 8));
   }
+  // kNorm: gamma of the lane's units (passes of one group share it)
+  constexpr int kPassesPerGroup = P >= 64 ? P / 64 : 1;
+  constexpr int kGamma = kNorm ? kStage / kPassesPerGroup : 1;
+  uint4 gamma[kGamma];
+  if constexpr (kNorm) {
+#pragma unroll
+    for (int i = 0; i < kGamma; ++i) {
+      const int g = wave + kW * pass_group(i * kPassesPerGroup);
+      gamma[i] = *reinterpret_cast<const uint4*>(p.norm_weight + g * G + wr * 8);
+    }
+  }
   __builtin_amdgcn_sched_barrier(0);
   Load buf[D];
 #pragma unroll
@@ -319,12 +349,58 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
     load_slab(buf[d], d);
     __builtin_amdgcn_sched_barrier(0);
   }
+  float inv_rms[kPassesPerGroup];  // of the lane's rows
+  if constexpr (kNorm) {
+    // Sums of squares of the wave's groups, per row: over the lane's units, the WR lanes of a row
+    // (and the two groups of a pass, P = 32), then the waves through LDS.
+    float* sq = sm.red + kW * MT * kSliceCols;  // [kW][MT]
+#pragma unroll
+    for (int q = 0; q < kPassesPerGroup; ++q) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int i = q; i < kStage; i += kPassesPerGroup) {
+        const int gi = P >= 64 ? (i * 64) / P : i * kGroupsPerPass + gsub;
+        const uint32_t words[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+        float s1 = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = act_bits_to_float<A>(static_cast<uint16_t>(words[e]));
+          const float hi = act_bits_to_float<A>(static_cast<uint16_t>(words[e] >> 16));
+          s1 = fmaf(hi, hi, fmaf(lo, lo, s1));
+        }
+        ss += gi <= g_last ? s1 : 0.0f;  // passes past the wave's groups repeat the last one
+      }
+      ss = group_sum<WR>(ss);
+      if constexpr (P < 64) {
+        ss += __shfl_xor(ss, 32);
+      }
+      sq[wave * MT + (P >= 64 ? q * 64 / WR : 0) + m_l] = ss;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < kPassesPerGroup; ++q) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kW; ++w) {
+        ss += sq[w * MT + (P >= 64 ? q * 64 / WR : 0) + m_l];
+      }
+      inv_rms[q] = 1.0f / sqrtf(ss / static_cast<float>(p.K) + p.eps);
+    }
+  }
   // Convert and store: rows past the batch stage zeros (a mask, not a branch); a pass past the
   // wave's last group stores that group's values again.
 #pragma unroll
   for (int i = 0; i < kStage; ++i) {
     const int g = wave + kW * pass_group(i);
     const int m = pass_row(i);
+    if constexpr (kNorm) {
+      const uint4 gw = gamma[i / kPassesPerGroup];
+      const float inv = inv_rms[i % kPassesPerGroup];
+      raw[i].x = norm_pair<A>(raw[i].x, gw.x, inv);
+      raw[i].y = norm_pair<A>(raw[i].y, gw.y, inv);
+      raw[i].z = norm_pair<A>(raw[i].z, gw.z, inv);
+      raw[i].w = norm_pair<A>(raw[i].w, gw.w, inv);
+    }
     const uint32_t keep = m < rows ? 0xffffffffu : 0u;
     uint4 v = make_uint4(raw[i].x & keep, raw[i].y & keep, raw[i].z & keep, raw[i].w & keep);
     float undo = 1.0f;
@@ -521,6 +597,7 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
       lds_barrier();
     }
   }
+  float gate[kSilu ? kPer : 1];  // kSilu: the pair whose turn it is, on the wave that writes it
   for (int r = 0; r < rg.whole; ++r) {
     const int n_loop = r == rg.whole - 1 ? nbs - 1 : nbs;
     for (int blk = 0; blk < n_loop; ++blk) {
@@ -530,7 +607,27 @@ __global__ void __launch_bounds__(64 * (kW + (kPieces ? 1 : 0)), 1)
       block_r((nbs - 1) * Q + wave, std::false_type{});
     }
     reduce();
-    if (wave == (r & (kW - 1))) {
+    if constexpr (kSilu) {
+      const int pair = r < pairs ? r : r - pairs;
+      if (wave == pair) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+          const int o = lane + 64 * i;
+          if (o < n_out) {
+            const float v = act_bits_to_float<A>(float_to_act_bits<A>(total(o)));
+            if (r < pairs) {
+              gate[i] = v;
+            } else {
+              const float act = act_bits_to_float<A>(
+                  float_to_act_bits<A>(gate[i] / (1.0f + expf(-gate[i]))));
+              p.out[static_cast<size_t>(o / kSliceCols) * (p.N / 2) +
+                    static_cast<size_t>(rg.whole_slice0 + pair) * kSliceCols + o % kSliceCols] =
+                  float_to_act_bits<A>(act * v);
+            }
+          }
+        }
+      }
+    } else if (wave == (r & (kW - 1))) {
       const size_t slice = static_cast<size_t>(rg.whole_slice0) + r;
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
@@ -602,6 +699,25 @@ hipError_t launch_mfma_stream_t(const GemvLaunch& l, hipStream_t stream) {
     }
     return hipErrorInvalidValue;
   }
+  if constexpr (is_native(F)) {
+    // (and the waves' row sums of squares, [waves][MT] floats)
+    const size_t fused_lds = lds + kStreamWaves * MT * sizeof(float);
+    auto launch = [&](auto fuse) {
+      hipLaunchKernelGGL((w4a16_gemm_mfma_stream_kernel<G, A, F, kStreamWaves, D, MT, false, false,
+                                                        decltype(fuse)::value>),
+                         dim3(grid), dim3(64 * kStreamWaves), fused_lds, stream, p);
+      return hipGetLastError();
+    };
+    switch (l.fuse) {
+      case GemvFuse::kNone: break;
+      case GemvFuse::kRmsNorm:
+        return launch(std::integral_constant<GemvFuse, GemvFuse::kRmsNorm>{});
+      case GemvFuse::kSiluMul:
+        return launch(std::integral_constant<GemvFuse, GemvFuse::kSiluMul>{});
+      case GemvFuse::kRmsNormSiluMul:
+        return launch(std::integral_constant<GemvFuse, GemvFuse::kRmsNormSiluMul>{});
+    }
+  }
   hipLaunchKernelGGL((w4a16_gemm_mfma_stream_kernel<G, A, F, kStreamWaves, D, MT, false>),
                      dim3(grid), dim3(64 * kStreamWaves), lds, stream, p);
   return hipGetLastError();
@@ -644,12 +760,21 @@ bool mfma_stream_fits(int group_size, int k, int batch) {
 
 hipError_t launch_w4a16_gemm_mfma_stream(const GemvLaunch& l, hipStream_t stream) {
   if (l.mode != GemvMode::kStreamK || !l.stream || l.m_tile != kMfmaRows || l.M < 1 ||
-      l.M > kMfmaRows || l.fuse != GemvFuse::kNone || l.slice_cols != kSliceCols ||
+      l.M > kMfmaRows || l.slice_cols != kSliceCols ||
       l.stream_half || l.stream_grid <= 0 || l.stream_parts < 1 ||
       (l.stream_parts == 1 && !mfma_stream_fits(l.group_size, l.K, l.M))) {
     return hipErrorInvalidValue;
   }
   const int ng = l.K / l.group_size;
+  if (l.fuse != GemvFuse::kNone) {
+    // whole slices (or gate and up slice pairs, one output wave each) of native slabs
+    const bool silu = l.fuse != GemvFuse::kRmsNorm;
+    if (!is_native(l.format) || l.stream_pieces || l.stream_parts != 1 ||
+        (l.fuse != GemvFuse::kSiluMul && l.norm_weight == nullptr) ||
+        (silu && (l.stream_whole % 2 != 0 || l.stream_whole > 2 * kStreamWaves))) {
+      return hipErrorInvalidValue;
+    }
+  }
   const int quantum = l.stream_waves * l.stream_depth;
   if (l.stream_waves != kStreamWaves ||
       l.stream_depth != stream_depth_for_kb(l.group_size, kStreamKB) || ng % quantum != 0) {

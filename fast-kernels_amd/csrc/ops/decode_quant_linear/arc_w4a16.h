@@ -143,6 +143,17 @@ void arc_w4a16_forward_silu_mul(std::uintptr_t activations_ptr, std::uintptr_t p
                                 std::uintptr_t stream_ptr, std::uintptr_t norm_weight_ptr = 0,
                                 float eps = 0.0f);
 
+// Both neighbours with a workspace, which lets them take every kernel they have: silu = false is
+// arc_w4a16_forward_rmsnorm (norm_weight_ptr not null), silu = true arc_w4a16_forward_silu_mul.
+// Workspace contract as arc_w4a16_forward_ex, plan_w4a16_fused's workspace_bytes.
+ArcW4A16Plan plan_w4a16_fused(int batch, int n, int k, int group_size, int activation_dtype,
+                              int cu_count, int packet_format, bool silu);
+void w4a16_forward_fused(std::uintptr_t activations_ptr, std::uintptr_t norm_weight_ptr, float eps,
+                         std::uintptr_t packets_ptr, std::uintptr_t output_ptr,
+                         std::uintptr_t workspace_ptr, std::size_t workspace_bytes, int batch,
+                         int n, int k, int group_size, int packet_format, int activation_dtype,
+                         bool silu, std::uintptr_t stream_ptr);
+
 // Bytes per packet of a format.
 int packet_format_stride_bytes(int group_size, int packet_format);
 

@@ -351,6 +351,27 @@ constexpr int kMfmaStreamMinBatch = 2;
 constexpr int kMfmaStreamMaxBatch = 16;
 constexpr int kMfmaPiecesMinBatch = 3;
 constexpr int kMfmaPiecesMaxBatch = 8;
+// Fused neighbours on the matrix-core stream kernel (us on MI355X, bf16 G128, dot2 runs -> this):
+// RMSNorm + 6144 x 4096 at 2 / 4 / 8 / 16 rows 8.8 -> 7.6, 12.7 -> 7.7, 20.5 -> 10.1, 38.3 -> 14.0;
+// RMSNorm + 28672 x 4096 + SiLU 21.5 -> 16.0, 38.6 -> 16.9, 65.6 -> 19.8, 128.9 -> 24.5. With fewer
+// than 64 slices only where the dot2 kernels' 8-row tiles are half empty or more than one: RMSNorm +
+// 1024 x 2048 at 2-4 rows 5.4-7.5 either way, at 8 rows 12.0 -> 8.5, at 16 rows 12.1 -> 12.4 (not
+// taken).
+constexpr long long kMfmaFusedMinSlices = 64;
+bool fused_mfma_takes_small(int batch, bool silu) {
+  return batch >= 5 && (batch <= 8 || silu);
+}
+// Fewest weights from which a fused neighbour that the stream kernels do not take (long K, slices
+// that do not divide) goes from the dot2 kernels to the row-tile GEMM, whose two launches take 13 us
+// at least: RMSNorm + 10240 x 8192 at 2 / 4 / 8 rows 19.2 / 29.2 / 68.9 us against 22.7 at any,
+// RMSNorm + 8192 x 11008 G64 + SiLU 34 / 54 / 94 against 26.8, 1024 x 2048 at 8-16 rows 12.0
+// against 13.1, 2048 x 4096 G64 at 8 rows 15.9 against 15.2.
+long long tile_fused_min_weights(int batch) {
+  return batch >= 17 ? 0 : batch >= 5 ? 4LL << 20 : batch >= 3 ? 32LL << 20 : 84LL << 20;
+}
+bool tile_takes_fused(int batch, int n, int k) {
+  return batch >= 2 && static_cast<long long>(n) * k >= tile_fused_min_weights(batch);
+}
 bool mfma_stream_enabled() {
   static const bool enabled = env_enabled("FK_W4A16_MFMA_STREAM");
   return enabled;
@@ -753,6 +774,54 @@ bool mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_siz
   return true;
 }
 
+// The fused decode-step neighbours on the matrix-core stream kernel: 2-16 rows of native slabs whose
+// rows stage whole, in whole slices (silu: pairs of a gate and the same up slice) over every CU, a
+// divisor grid, or one unit per workgroup.
+bool fused_mfma_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool silu,
+                     int cu_count, bool cu_count_given) {
+  if (batch < kMfmaStreamMinBatch || batch > kMfmaStreamMaxBatch || !mfma_stream_enabled() ||
+      !stream_fused_enabled()) {
+    return false;
+  }
+  const int depth = fk::stream_depth_for_kb(group_size, fk::kStreamKB);
+  const int num_groups = k / group_size;
+  const std::size_t lds_limit = cu_count_given ? kGfx950LdsBytes : device_lds_per_block();
+  const std::size_t row_sums = static_cast<std::size_t>(fk::kStreamWaves) * fk::kMfmaRows * sizeof(float);
+  const long long slices = n / fk::kSliceCols;
+  if (num_groups % (fk::kStreamWaves * depth) != 0 ||
+      !fk::mfma_stream_fits(group_size, k, batch) ||
+      fk::mfma_stream_lds(group_size, k, batch) + row_sums > lds_limit) {
+    return false;
+  }
+  if (slices < kMfmaFusedMinSlices && !fused_mfma_takes_small(batch, silu)) {
+    return false;
+  }
+  const long long units = silu ? slices / 2 : slices;
+  const long long cus = cu_count;
+  long long grid = 0;
+  if (units % cus == 0) {
+    grid = cus;
+  } else if (const long long dgrid = divisor_grid(units, cus); dgrid > 0) {
+    grid = dgrid;
+  } else if (units < cus) {
+    grid = units;
+  }
+  // (one wave writes a pair: at most as many pairs as waves)
+  if (grid == 0 || (silu && units / grid > fk::kStreamWaves)) {
+    return false;
+  }
+  plan = ArcW4A16Plan{};
+  plan.m_tile = fk::kMfmaRows;
+  plan.schedule = kScheduleStream;
+  plan.slice_cols = fk::kSliceCols;
+  plan.workgroups = static_cast<int>(grid);
+  plan.stream_depth = depth;
+  plan.stream_whole = static_cast<int>(units / grid) * (silu ? 2 : 1);
+  plan.groups_per_workgroup = plan.stream_whole * num_groups;
+  plan.max_tile_contributors = 1;
+  return true;
+}
+
 // The reference-signature plan's matrix-core stream schedule over the reference packets (the
 // automatic kernel choice).
 bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size,
@@ -1120,7 +1189,9 @@ void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::u
     const int cols = plan.stream_half ? fk::kSliceCols / 2 : fk::kSliceCols;
     const bool rows_ok = plan.m_tile == fk::kMfmaRows ? batch <= fk::kMfmaRows : plan.m_tile == batch;
     if (format == fk::PacketFormat::kArc || !rows_ok || plan.slice_cols != cols ||
-        (fuse != fk::GemvFuse::kNone && (batch != 1 || plan.stream_pieces || plan.stream_half))) {
+        (fuse != fk::GemvFuse::kNone &&
+         ((batch != 1 && plan.m_tile != fk::kMfmaRows) || plan.stream_pieces || plan.stream_half ||
+          plan.max_tile_contributors != 1))) {
       throw std::logic_error("stream schedule on a plan the stream kernel does not take");
     }
     l.stream = true;
@@ -1179,6 +1250,19 @@ void validate_forward_buffers(std::uintptr_t activations_ptr, std::uintptr_t pac
   validate_pointer(activations_ptr, 16, "activations");
   validate_pointer(packets_ptr, 16, "packets");
   validate_pointer(output_ptr, 2, "output");
+}
+
+void validate_workspace(const ArcW4A16Plan& plan, std::uintptr_t workspace_ptr,
+                        std::size_t workspace_bytes) {
+  if (plan.workspace_bytes > 0) {
+    validate_pointer(workspace_ptr, kCounterRegionAlign, "workspace");
+    if (workspace_bytes < plan.workspace_bytes) {
+      std::ostringstream oss;
+      oss << "workspace_bytes=" << workspace_bytes << " is smaller than the " << plan.workspace_bytes
+          << " bytes this launch needs";
+      throw_invalid(oss.str());
+    }
+  }
 }
 
 // ---- vendor baseline: dequantised fp16 weight x hipBLASLt --------------------------------
@@ -1468,15 +1552,7 @@ void forward_with_format(std::uintptr_t activations_ptr, std::uintptr_t packets_
   const ArcW4A16Plan plan =
       plan_w4a16_for_kernel(batch, n, k, group_size, activation_dtype, split_k_slices,
                             device_cu_count(), static_cast<int>(format), kernel);
-  if (plan.workspace_bytes > 0) {
-    validate_pointer(workspace_ptr, kCounterRegionAlign, "workspace");
-    if (workspace_bytes < plan.workspace_bytes) {
-      std::ostringstream oss;
-      oss << "workspace_bytes=" << workspace_bytes << " is smaller than the " << plan.workspace_bytes
-          << " bytes this launch needs";
-      throw_invalid(oss.str());
-    }
-  }
+  validate_workspace(plan, workspace_ptr, workspace_bytes);
   if (plan.schedule == kScheduleTiles) {
     run_tiles(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr),
               batch, n, k, group_size, activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr),
@@ -1651,15 +1727,7 @@ void arc_w4a16_forward_rmsnorm(std::uintptr_t activations_ptr, std::uintptr_t no
   }
   const ArcW4A16Plan plan = plan_w4a16_rmsnorm(batch, n, k, group_size, activation_dtype,
                                                split_k_slices, 0, packet_format);
-  if (plan.workspace_bytes > 0) {
-    validate_pointer(workspace_ptr, kCounterRegionAlign, "workspace");
-    if (workspace_bytes < plan.workspace_bytes) {
-      std::ostringstream oss;
-      oss << "workspace_bytes=" << workspace_bytes << " is smaller than the " << plan.workspace_bytes
-          << " bytes this launch needs";
-      throw_invalid(oss.str());
-    }
-  }
+  validate_workspace(plan, workspace_ptr, workspace_bytes);
   run_gemv(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr), plan,
            batch, n, k, group_size, activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr),
            format, fk::GemvFuse::kRmsNorm, norm_weight_ptr, eps);
@@ -1677,6 +1745,53 @@ ArcW4A16Plan plan_w4a16_rmsnorm(int batch, int n, int k, int group_size, int act
                               packet_format, kKernelDot2, /*plain=*/false);
 }
 
+namespace {
+
+// Plan of the SiLU-and-multiply call. One row: the stream kernel over whole (gate slice, up slice)
+// pairs where they divide over the CUs; 2-16 rows: the matrix-core stream kernel likewise; then,
+// where the caller brings a workspace, the row-tile GEMM. Otherwise one dot2 workgroup per pair
+// over all of K.
+ArcW4A16Plan silu_mul_plan(int batch, int n, int k, int group_size, int cu_count,
+                           bool with_workspace) {
+  ArcW4A16Plan plan{};
+  if (fused_stream_plan(plan, batch, n, k, group_size, /*silu=*/true, cu_count)) {
+    return plan;
+  }
+  const bool given = cu_count > 0;
+  const int cus = given ? cu_count : device_cu_count();
+  if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/true, cus, given)) {
+    return plan;
+  }
+  if (with_workspace && tile_takes_fused(batch, n, k) &&
+      tile_plan(plan, batch, n, k, group_size, /*silu=*/true, cus)) {
+    return plan;
+  }
+  plan = ArcW4A16Plan{};
+  plan.m_tile = fk::gemv_partials_m_tile_for_batch(batch);
+  plan.slice_cols = fk::kSliceCols;
+  plan.groups_per_workgroup = k / group_size;
+  plan.max_tile_contributors = 1;
+  return plan;
+}
+
+void validate_fused(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
+                    std::uintptr_t output_ptr, std::uintptr_t norm_weight_ptr, float eps, int n,
+                    int activation_dtype, bool silu) {
+  if (silu && n % (2 * fk::kTileCols) != 0) {
+    throw_invalid("n (gate and up rows together) must be divisible by 256");
+  }
+  validate_activation_dtype(activation_dtype);
+  validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
+  if (norm_weight_ptr != 0) {
+    if (!(eps >= 0.0f)) {
+      throw_invalid("eps must be >= 0");
+    }
+    validate_pointer(norm_weight_ptr, 16, "norm_weight");
+  }
+}
+
+}  // namespace
+
 void arc_w4a16_forward_silu_mul(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
                                 std::uintptr_t output_ptr, int batch, int n, int k, int group_size,
                                 int packet_format, int activation_dtype,
@@ -1687,29 +1802,69 @@ void arc_w4a16_forward_silu_mul(std::uintptr_t activations_ptr, std::uintptr_t p
     throw_invalid("n (gate and up rows together) must be divisible by 256");
   }
   const fk::PacketFormat format = to_packet_format(packet_format, false);
-  validate_activation_dtype(activation_dtype);
-  validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
-  const bool norm = norm_weight_ptr != 0;
-  if (norm && !(eps >= 0.0f)) {
-    throw_invalid("eps must be >= 0");
-  }
-  if (norm) {
-    validate_pointer(norm_weight_ptr, 16, "norm_weight");
-  }
-  // One row: the stream kernel over whole (gate slice, up slice) pairs where they divide over the
-  // CUs (fused_stream_plan). Otherwise one workgroup per pair over all of K. No fix-up, no
-  // workspace either way.
-  ArcW4A16Plan plan{};
-  if (!fused_stream_plan(plan, batch, n, k, group_size, /*silu=*/true, 0)) {
-    plan.m_tile = fk::gemv_partials_m_tile_for_batch(batch);
-    plan.slice_cols = fk::kSliceCols;
-    plan.groups_per_workgroup = k / group_size;
-    plan.max_tile_contributors = 1;
-    plan.workspace_bytes = 0;
-  }
+  validate_fused(activations_ptr, packets_ptr, output_ptr, norm_weight_ptr, eps, n,
+                 activation_dtype, /*silu=*/true);
+  const ArcW4A16Plan plan = silu_mul_plan(batch, n, k, group_size, 0, /*with_workspace=*/false);
   run_gemv(activations_ptr, packets_ptr, output_ptr, nullptr, plan, batch, n, k, group_size,
            activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr), format,
-           norm ? fk::GemvFuse::kRmsNormSiluMul : fk::GemvFuse::kSiluMul, norm_weight_ptr, eps);
+           norm_weight_ptr != 0 ? fk::GemvFuse::kRmsNormSiluMul : fk::GemvFuse::kSiluMul,
+           norm_weight_ptr, eps);
+}
+
+ArcW4A16Plan plan_w4a16_fused(int batch, int n, int k, int group_size, int activation_dtype,
+                              int cu_count, int packet_format, bool silu) {
+  validate_dimensions(batch, n, k, group_size);
+  validate_activation_dtype(activation_dtype);
+  to_packet_format(packet_format, false);
+  if (silu) {
+    if (n % (2 * fk::kTileCols) != 0) {
+      throw_invalid("n (gate and up rows together) must be divisible by 256");
+    }
+    return silu_mul_plan(batch, n, k, group_size, cu_count, /*with_workspace=*/true);
+  }
+  ArcW4A16Plan plan{};
+  if (fused_stream_plan(plan, batch, n, k, group_size, /*silu=*/false, cu_count)) {
+    return plan;
+  }
+  const bool given = cu_count > 0;
+  const int cus = given ? cu_count : device_cu_count();
+  if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/false, cus, given)) {
+    return plan;
+  }
+  if (tile_takes_fused(batch, n, k) &&
+      tile_plan(plan, batch, n, k, group_size, /*silu=*/false, cus)) {
+    return plan;
+  }
+  return plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, cu_count,
+                              packet_format, kKernelDot2, /*plain=*/false);
+}
+
+void w4a16_forward_fused(std::uintptr_t activations_ptr, std::uintptr_t norm_weight_ptr, float eps,
+                         std::uintptr_t packets_ptr, std::uintptr_t output_ptr,
+                         std::uintptr_t workspace_ptr, std::size_t workspace_bytes, int batch,
+                         int n, int k, int group_size, int packet_format, int activation_dtype,
+                         bool silu, std::uintptr_t stream_ptr) {
+  validate_dimensions(batch, n, k, group_size);
+  const fk::PacketFormat format = to_packet_format(packet_format, false);
+  validate_fused(activations_ptr, packets_ptr, output_ptr, norm_weight_ptr, eps, n,
+                 activation_dtype, silu);
+  if (!silu && norm_weight_ptr == 0) {
+    throw_invalid("norm_weight must not be null");
+  }
+  const ArcW4A16Plan plan =
+      plan_w4a16_fused(batch, n, k, group_size, activation_dtype, 0, packet_format, silu);
+  validate_workspace(plan, workspace_ptr, workspace_bytes);
+  const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  if (plan.schedule == kScheduleTiles) {
+    run_tiles(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr),
+              batch, n, k, group_size, activation_dtype, stream, format, silu, norm_weight_ptr, eps);
+    return;
+  }
+  const fk::GemvFuse fuse = !silu                   ? fk::GemvFuse::kRmsNorm
+                            : norm_weight_ptr != 0 ? fk::GemvFuse::kRmsNormSiluMul
+                                                   : fk::GemvFuse::kSiluMul;
+  run_gemv(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr), plan,
+           batch, n, k, group_size, activation_dtype, stream, format, fuse, norm_weight_ptr, eps);
 }
 
 }  // namespace fast_kernels::decode_quant_linear

@@ -289,6 +289,15 @@ def arc_w4a16_forward_rmsnorm(
         raise ValueError("split_k_slices must be positive")
     requested = 0 if split_k_slices is None else int(split_k_slices)
     act = _act_code(activations.dtype)
+    if requested == 0:
+        plan = native.w4a16_plan_fused(batch, n, k, group_size, act, 0, code, False)
+        _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+        native.w4a16_forward_fused(
+            activations.data_ptr(), norm_weight.data_ptr(), float(eps), packets.data_ptr(),
+            output.data_ptr(), ws_ptr, ws_bytes, batch, n, k, group_size, code, act, False,
+            _current_stream_ptr(activations.device),
+        )
+        return output
     plan = native.w4a16_plan_rmsnorm(batch, n, k, group_size, act, requested, 0, code)
     _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
     native.w4a16_forward_rmsnorm(
@@ -345,9 +354,12 @@ def arc_w4a16_forward_silu_mul(
             raise ValueError("norm_weight.shape[0] must match k")
         _check_same_device(("activations", activations), ("norm_weight", norm_weight))
         norm_ptr = norm_weight.data_ptr()
-    native.w4a16_forward_silu_mul(
-        activations.data_ptr(), packets.data_ptr(), output.data_ptr(), batch, n, k, group_size,
-        code, _act_code(activations.dtype), norm_ptr, float(eps),
+    act = _act_code(activations.dtype)
+    plan = native.w4a16_plan_fused(batch, n, k, group_size, act, 0, code, True)
+    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+    native.w4a16_forward_fused(
+        activations.data_ptr(), norm_ptr, float(eps), packets.data_ptr(), output.data_ptr(),
+        ws_ptr, ws_bytes, batch, n, k, group_size, code, act, True,
         _current_stream_ptr(activations.device),
     )
     return output

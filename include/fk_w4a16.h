@@ -269,6 +269,17 @@ int fk_w4a16_forward_silu_mul(const void* activations, const void* packets, void
                               int activation_dtype, const void* norm_weight, float eps,
                               void* stream);
 
+/* Both fused neighbours with a workspace (workspace_bytes from fk_w4a16_plan_fused, contract of
+ * fk_arc_w4a16_forward_ex), which lets several rows run on the matrix cores where the calls above
+ * keep the dot2 kernels: silu = 0 is fk_w4a16_forward_rmsnorm (norm_weight not NULL), silu = 1
+ * fk_w4a16_forward_silu_mul. Same results up to the order of the fp32 sums. */
+int fk_w4a16_plan_fused(int batch, int n, int k, int group_size, int activation_dtype,
+                        int cu_count, int packet_format, int silu, fk_arc_w4a16_plan* plan);
+int fk_w4a16_forward_fused(const void* activations, const void* norm_weight, float eps,
+                           const void* packets, void* output, void* workspace,
+                           size_t workspace_bytes, int batch, int n, int k, int group_size,
+                           int packet_format, int activation_dtype, int silu, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
