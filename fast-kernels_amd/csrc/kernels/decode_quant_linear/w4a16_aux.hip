@@ -17,39 +17,12 @@ namespace {
 
 constexpr int kAuxThreads = 256;
 
-// pack_arc_packets_kernel (arc_w4a16.cu:87-122): packet (tile, g) holds word w of column c at
-// byte (w*128 + c)*4, then alpha[128], then beta[128] (fp16). One thread per (tile, g, column):
-// it reads its G/2 code bytes as 16-byte vectors and writes G/8 words; lanes of a wave write
-// consecutive columns, so every store instruction covers 256 contiguous bytes.
-template <int G>
-__global__ void __launch_bounds__(kTileCols)
-pack_packets_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ alpha,
-                    const uint16_t* __restrict__ beta, uint8_t* __restrict__ packets, int k,
-                    int num_groups) {
-  constexpr int kGroupBytes = G / 2;
-  constexpr int kVecs = kGroupBytes / 16;
-  constexpr int QB = kTileCols * kGroupBytes;
-  const int tile = static_cast<int>(blockIdx.x);
-  const int g = static_cast<int>(blockIdx.y);
-  const int c = static_cast<int>(threadIdx.x);
-  const size_t row = static_cast<size_t>(tile) * kTileCols + c;
-  const size_t stride = static_cast<size_t>(packet_stride_bytes(G));
-  uint8_t* packet = packets + (static_cast<size_t>(tile) * num_groups + g) * stride;
-  const uint4* src = reinterpret_cast<const uint4*>(q + row * (k / 2) + static_cast<size_t>(g) * kGroupBytes);
-  uint32_t* words = reinterpret_cast<uint32_t*>(packet);
-#pragma unroll
-  for (int v = 0; v < kVecs; ++v) {
-    const uint4 d = src[v];
-    words[(4 * v + 0) * kTileCols + c] = d.x;
-    words[(4 * v + 1) * kTileCols + c] = d.y;
-    words[(4 * v + 2) * kTileCols + c] = d.z;
-    words[(4 * v + 3) * kTileCols + c] = d.w;
-  }
-  uint16_t* a_dst = reinterpret_cast<uint16_t*>(packet + QB);
-  uint16_t* b_dst = a_dst + kTileCols;
-  a_dst[c] = alpha[row * num_groups + g];
-  b_dst[c] = beta[row * num_groups + g];
-}
+// Code words of one 128-row tile over 256 values of K in LDS, word row by word row as in a reference
+// packet; the pitch keeps rows 16-byte aligned and spreads the word rows over the banks.
+constexpr int kTurnK = 256;
+constexpr int kTurnWords = kTurnK / 8;
+constexpr int kTurnPitch = kTileCols + 4;
+constexpr int kMaxTurns = 4;  // turns of 256 values a packing workgroup takes at most
 
 // half_rn(fma(alpha, q, beta)) for the 8 codes of one uint32 word (k = 8w .. 8w+7). For the
 // quantisation recipes used here alpha*q + beta is exact in fp32, so the single fp16 rounding
@@ -83,29 +56,54 @@ dequant_kernel(const uint32_t* __restrict__ q, const uint16_t* __restrict__ alph
   out[idx] = dequant_word(q[idx], a, b);
 }
 
-// dequant_arc_packets_kernel (arc_w4a16.cu:183-220): packets -> W[N, K] fp16. One thread per
-// (row, word); consecutive threads take consecutive words of a row so the 16-byte stores are
-// contiguous.
+// dequant_arc_packets_kernel (arc_w4a16.cu:183-220): packets -> W[N, K] fp16. A workgroup takes a
+// tile over 256 values of K: 512-byte word rows in, through LDS, 512 bytes of each row of W out
+// (a row's words are 512 bytes apart in the packets: reading them in W's order fetched every line
+// many times over). HBM-bound: 8192 x 8192 G128 69.3 -> 29.6 us back to back (5.8 TB/s; a large copy
+// runs at 5.2), 28672 x 4096 117.5 -> 54.8.
 template <int G>
 __global__ void __launch_bounds__(kAuxThreads)
-dequant_packets_kernel(const uint8_t* __restrict__ packets, uint4* __restrict__ out,
-                       size_t total_words, int words_per_row, int num_groups) {
+dequant_packets_kernel(const uint8_t* __restrict__ packets, uint4* __restrict__ out, int k,
+                       int num_groups) {
   constexpr int QB = kTileCols * G / 2;
-  const size_t idx = static_cast<size_t>(blockIdx.x) * kAuxThreads + threadIdx.x;
-  if (idx >= total_words) {
-    return;
+  constexpr int WR = G / 8;
+  constexpr int kGroups = kTurnK / G;
+  __shared__ __attribute__((aligned(16))) uint32_t words[kTurnWords][kTurnPitch];
+  __shared__ uint16_t scales[kGroups][2 * kTileCols];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int tile = static_cast<int>(blockIdx.y);
+  const int g0 = static_cast<int>(blockIdx.x) * kGroups;
+  const int groups = min(kGroups, num_groups - g0);
+  const size_t stride = static_cast<size_t>(packet_stride_bytes(G));
+  const uint8_t* src = packets + (static_cast<size_t>(tile) * num_groups + g0) * stride;
+#pragma unroll
+  for (int it = 0; it < kTurnWords * kTileCols / 4 / kAuxThreads; ++it) {
+    const int u = it * kAuxThreads + tid;
+    const int wr = u / (kTileCols / 4);
+    const int c = u % (kTileCols / 4) * 4;
+    if (wr < groups * WR) {
+      *reinterpret_cast<uint4*>(&words[wr][c]) =
+          stream_load16(src + (wr / WR) * stride + (wr % WR * kTileCols + c) * 4);
+    }
   }
-  const size_t row = idx / words_per_row;
-  const int w = static_cast<int>(idx % words_per_row);
-  const int g = (w * 8) / G;
-  const int wg = w % (G / 8);
-  const size_t tile = row / kTileCols;
-  const int c = static_cast<int>(row % kTileCols);
-  const uint8_t* packet =
-      packets + (tile * num_groups + g) * static_cast<size_t>(packet_stride_bytes(G));
-  const uint32_t word = reinterpret_cast<const uint32_t*>(packet)[wg * kTileCols + c];
-  const uint16_t* ab = reinterpret_cast<const uint16_t*>(packet + QB);
-  out[idx] = dequant_word(word, half_bits_to_float(ab[c]), half_bits_to_float(ab[kTileCols + c]));
+  for (int i = tid; i < groups * kTileCols; i += kAuxThreads) {  // two scales a thread
+    const int g = i / kTileCols;
+    reinterpret_cast<uint32_t*>(scales[g])[i % kTileCols] =
+        reinterpret_cast<const uint32_t*>(src + g * stride + QB)[i % kTileCols];
+  }
+  __syncthreads();
+  const int words_per_row = k / 8;
+#pragma unroll 4
+  for (int it = 0; it < kTurnWords * kTileCols / kAuxThreads; ++it) {
+    const int u = it * kAuxThreads + tid;
+    const int c = u / kTurnWords;
+    const int wr = u % kTurnWords;
+    if (wr < groups * WR) {
+      const uint16_t* ab = scales[wr / WR];
+      out[(static_cast<size_t>(tile) * kTileCols + c) * words_per_row + g0 * WR + wr] = dequant_word(
+          words[wr][c], half_bits_to_float(ab[c]), half_bits_to_float(ab[kTileCols + c]));
+    }
+  }
 }
 
 // compute_arc_group_sums_kernel (arc_w4a16.cu:124-158): sums[b, g] = sum of x[b, g*G .. +G) in
@@ -194,32 +192,126 @@ __device__ __forceinline__ void store_neg_zp(NativeSlot s, uint32_t zp) {
   reinterpret_cast<uint16_t*>(slab_zp_word<G>(s))[s.i] = neg_zp_half_bits(zp & 0xFu);
 }
 
-// Native slabs from q_u8 / alpha / zero points (uint8 [N, NG], values 0..15, unused for
-// kNativeSym). One thread per column of a (tile, group).
+// Packets of any format from q_u8 [N, K/2], alpha [N, NG] and the offsets: beta fp16 (kArc,
+// pack_arc_packets_kernel, arc_w4a16.cu:87-122: word w of column c at byte (w*128 + c)*4, then
+// alpha[128], then beta[128]) or zero points uint8 [N, NG], values 0..15 (kNativeAsym). A workgroup
+// takes a tile, 256 values of K at a time: 128 bytes of each of the tile's rows in, through LDS,
+// whole word rows (kArc) or 1 KB runs of slabs out; scales through LDS too, those of up to four
+// turns at once. (One thread per column and group read 64 bytes of each row, with the line's other
+// half read by another workgroup much later, and every scale with a line of its own.) HBM-bound:
+// 28672 x 4096 to reference packets G128 31.0 -> 26.7 us (4.7 TB/s), G64 42.1 -> 33.1; to native
+// slabs 28.9 -> 24.0 and 34.7 -> 26.8.
 template <int G, PacketFormat F>
-__global__ void __launch_bounds__(kTileCols)
-pack_native_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ alpha,
-                   const uint8_t* __restrict__ zero_points, uint8_t* __restrict__ packets, int k,
-                   int num_groups) {
-  constexpr int kGroupBytes = G / 2;
-  constexpr int kVecs = kGroupBytes / 16;
-  const int tile = static_cast<int>(blockIdx.x);
-  const int g = static_cast<int>(blockIdx.y);
-  const int c = static_cast<int>(threadIdx.x);
-  const size_t row = static_cast<size_t>(tile) * kTileCols + c;
-  const NativeSlot s = native_slot<G, F>(packets, tile, g, c, num_groups);
-  const uint4* src = reinterpret_cast<const uint4*>(q + row * (k / 2) + static_cast<size_t>(g) * kGroupBytes);
-#pragma unroll
-  for (int v = 0; v < kVecs; ++v) {
-    const uint4 d = src[v];
-    *slab_word<G>(s, 4 * v + 0) = d.x;
-    *slab_word<G>(s, 4 * v + 1) = d.y;
-    *slab_word<G>(s, 4 * v + 2) = d.z;
-    *slab_word<G>(s, 4 * v + 3) = d.w;
+__global__ void __launch_bounds__(kAuxThreads)
+pack_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ alpha,
+            const void* __restrict__ offsets, uint8_t* __restrict__ packets, int k, int num_groups,
+            int turns_per_group) {
+  constexpr int WR = G / 8;
+  constexpr int kGroups = kTurnK / G;
+  constexpr size_t kStride = format_packet_stride(G, F);
+  constexpr bool kOffsets = F != PacketFormat::kNativeSym;
+  constexpr int kScalePitch = kTileCols + 2;  // 4-byte aligned, groups on different banks
+  __shared__ __attribute__((aligned(16))) uint32_t words[kTurnWords][kTurnPitch];
+  __shared__ __attribute__((aligned(4))) uint16_t scales[kOffsets ? 2 : 1][kMaxTurns * kGroups][kScalePitch];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int tile = static_cast<int>(blockIdx.y);
+  const size_t row0 = static_cast<size_t>(tile) * kTileCols;
+  const int turns = (num_groups + kGroups - 1) / kGroups;
+  const int turn0 = static_cast<int>(blockIdx.x) * turns_per_group;
+  const int turn1 = min(turns, turn0 + turns_per_group);
+  // Group g of the tile: its packet (kArc), or its slab of slice s.
+  auto packet = [&](int s, int g) {
+    const size_t unit = F == PacketFormat::kArc ? static_cast<size_t>(tile)
+                                                : static_cast<size_t>(tile) * kSlicesPerTile + s;
+    return packets + (unit * num_groups + g) * kStride;
+  };
+  // The workgroup's scales first, consecutive lanes on consecutive groups of a row.
+  const int first = turn0 * kGroups;
+  const int width = turns_per_group * kGroups;  // a power of two
+  const int shift = __builtin_ctz(width);
+  const int have = min(num_groups - first, width);
+  for (int i = tid; i < kTileCols << shift; i += kAuxThreads) {
+    const int c = i >> shift;
+    const int g = i & (width - 1);
+    if (g < have) {
+      const size_t at = (row0 + c) * num_groups + first + g;
+      scales[0][g][c] = alpha[at];
+      if constexpr (F == PacketFormat::kArc) {
+        scales[1][g][c] = static_cast<const uint16_t*>(offsets)[at];
+      } else if constexpr (kOffsets) {
+        scales[1][g][c] = neg_zp_half_bits(static_cast<const uint8_t*>(offsets)[at] & 0xFu);
+      }
+    }
   }
-  *slab_alpha<G, F>(s) = alpha[row * num_groups + g];
-  if constexpr (F == PacketFormat::kNativeAsym) {
-    store_neg_zp<G>(s, zero_points[row * num_groups + g]);
+  for (int turn = turn0; turn < turn1; ++turn) {
+    const int g0 = turn * kGroups;
+    const int groups = min(kGroups, num_groups - g0);
+    if (turn != turn0) {
+      __syncthreads();
+    }
+    const uint8_t* src = q + row0 * (k / 2) + static_cast<size_t>(g0) * (G / 2);
+#pragma unroll
+    for (int it = 0; it < kTurnWords * kTileCols / 4 / kAuxThreads; ++it) {
+      const int u = it * kAuxThreads + tid;
+      const int v = u % (kTurnWords / 4);
+      const int r = u / (kTurnWords / 4);
+      if (4 * v < groups * WR) {
+        const uint4 d = stream_load16(src + static_cast<size_t>(r) * (k / 2) + v * 16);
+        words[4 * v + 0][r] = d.x;
+        words[4 * v + 1][r] = d.y;
+        words[4 * v + 2][r] = d.z;
+        words[4 * v + 3][r] = d.w;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kTurnWords * kTileCols / 4 / kAuxThreads; ++it) {
+      const int u = it * kAuxThreads + tid;
+      constexpr int kUnits = WR * kTileCols / 4;  // 16-byte units of a group
+      const int g = u / kUnits;
+      const int e = u % kUnits;
+      if (g < groups) {
+        if constexpr (F == PacketFormat::kArc) {
+          const uint4 d = *reinterpret_cast<const uint4*>(&words[g * WR + e / 32][e % 32 * 4]);
+          *reinterpret_cast<uint4*>(packet(0, g0 + g) + e * 16) = d;
+        } else {
+          // unit l of half i (G = 128), or both halves' two words (G = 64), of slice s
+          constexpr int kPerSlice = kUnits / kSlicesPerTile;
+          const int s = e / kPerSlice;
+          const int l = e % 64;
+          const int n = s * kSliceCols + l % 16;
+          const int w0 = g * WR + l / 16 * native_unit_words(G);
+          uint4 d;
+          if constexpr (G == 128) {
+            const int c = n + 16 * (e % kPerSlice / 64);
+            d = make_uint4(words[w0][c], words[w0 + 1][c], words[w0 + 2][c], words[w0 + 3][c]);
+          } else {
+            d = make_uint4(words[w0][n], words[w0 + 1][n], words[w0][n + 16], words[w0 + 1][n + 16]);
+          }
+          *reinterpret_cast<uint4*>(packet(s, g0 + g) + e % kPerSlice * 16) = d;
+        }
+      }
+    }
+    // scales, 4 bytes a store: two columns' alphas or betas (kArc), a record or half of one
+    for (int i = tid; i < groups * kTileCols; i += kAuxThreads) {
+      const int g = i / kTileCols;
+      const int e = i % kTileCols;
+      const int gs = g0 - first + g;
+      if constexpr (F == PacketFormat::kArc) {
+        const int c = 2 * e % kTileCols;
+        reinterpret_cast<uint32_t*>(packet(0, g0 + g) + kTileCols * G / 2)[e] =
+            *reinterpret_cast<const uint32_t*>(&scales[2 * e / kTileCols][gs][c]);
+      } else {
+        constexpr int kWords = native_record_bytes(F) / 4;
+        const int s = e / (16 * kWords);
+        const int n = e / kWords % 16;
+        if (s < kSlicesPerTile) {
+          const uint16_t* row = scales[kOffsets ? e % kWords : 0][gs] + s * kSliceCols + n;
+          reinterpret_cast<uint32_t*>(packet(s, g0 + g) + native_record_offset(G))[e % (16 * kWords)] =
+              row[0] | (static_cast<uint32_t>(row[16]) << 16);
+        }
+      }
+    }
   }
 }
 
@@ -293,20 +385,33 @@ native_to_arc_kernel(const uint8_t* __restrict__ native, uint8_t* __restrict__ a
 
 }  // namespace
 
+namespace {
+
+// Turns (256 values of K) per workgroup: up to 4, so that a row's scales are read by few
+// workgroups, while at least 4 workgroups per CU remain.
+template <int G, PacketFormat F>
+hipError_t launch_pack(const void* q, const void* alpha, const void* offsets, void* packets, int n,
+                       int k, hipStream_t stream) {
+  const int tiles = n / kTileCols;
+  const int turns = (k + kTurnK - 1) / kTurnK;
+  int per = kMaxTurns;
+  while (per > 1 && static_cast<long long>(tiles) * ((turns + per - 1) / per) < 1024) {
+    per /= 2;
+  }
+  const dim3 grid(static_cast<unsigned int>((turns + per - 1) / per), static_cast<unsigned int>(tiles));
+  hipLaunchKernelGGL((pack_kernel<G, F>), grid, dim3(kAuxThreads), 0, stream,
+                     static_cast<const uint8_t*>(q), static_cast<const uint16_t*>(alpha), offsets,
+                     static_cast<uint8_t*>(packets), k, k / G, per);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_pack_packets(const void* q, const void* alpha, const void* beta, void* packets,
                                int n, int k, int group_size, hipStream_t stream) {
-  const int num_groups = k / group_size;
-  const dim3 grid(static_cast<unsigned int>(n / kTileCols), static_cast<unsigned int>(num_groups));
-  auto* qp = static_cast<const uint8_t*>(q);
-  auto* ap = static_cast<const uint16_t*>(alpha);
-  auto* bp = static_cast<const uint16_t*>(beta);
-  auto* pp = static_cast<uint8_t*>(packets);
-  if (group_size == 64) {
-    hipLaunchKernelGGL(pack_packets_kernel<64>, grid, dim3(kTileCols), 0, stream, qp, ap, bp, pp, k, num_groups);
-  } else {
-    hipLaunchKernelGGL(pack_packets_kernel<128>, grid, dim3(kTileCols), 0, stream, qp, ap, bp, pp, k, num_groups);
-  }
-  return hipGetLastError();
+  return group_size == 64
+             ? launch_pack<64, PacketFormat::kArc>(q, alpha, beta, packets, n, k, stream)
+             : launch_pack<128, PacketFormat::kArc>(q, alpha, beta, packets, n, k, stream);
 }
 
 hipError_t launch_dequant(const void* q, const void* alpha, const void* beta, void* out, int n,
@@ -330,17 +435,15 @@ hipError_t launch_dequant(const void* q, const void* alpha, const void* beta, vo
 
 hipError_t launch_dequant_packets(const void* packets, void* out, int n, int k, int group_size,
                                   hipStream_t stream) {
-  const int words_per_row = k / 8;
-  const size_t total = static_cast<size_t>(n) * words_per_row;
   const int num_groups = k / group_size;
+  const dim3 grid(static_cast<unsigned int>((k + kTurnK - 1) / kTurnK),
+                  static_cast<unsigned int>(n / kTileCols));
   auto* pp = static_cast<const uint8_t*>(packets);
   auto* op = static_cast<uint4*>(out);
   if (group_size == 64) {
-    hipLaunchKernelGGL(dequant_packets_kernel<64>, dim3(blocks_for(total, kAuxThreads)), dim3(kAuxThreads), 0,
-                       stream, pp, op, total, words_per_row, num_groups);
+    hipLaunchKernelGGL(dequant_packets_kernel<64>, grid, dim3(kAuxThreads), 0, stream, pp, op, k, num_groups);
   } else {
-    hipLaunchKernelGGL(dequant_packets_kernel<128>, dim3(blocks_for(total, kAuxThreads)), dim3(kAuxThreads), 0,
-                       stream, pp, op, total, words_per_row, num_groups);
+    hipLaunchKernelGGL(dequant_packets_kernel<128>, grid, dim3(kAuxThreads), 0, stream, pp, op, k, num_groups);
   }
   return hipGetLastError();
 }
@@ -371,23 +474,16 @@ hipError_t launch_reduce_partials(const void* partials, void* out, int batch, in
 hipError_t launch_pack_native(const void* q, const void* alpha, const void* zero_points,
                               void* packets, int n, int k, int group_size, PacketFormat format,
                               hipStream_t stream) {
-  const int ng = k / group_size;
-  const dim3 grid(static_cast<unsigned int>(n / kTileCols), static_cast<unsigned int>(ng));
-  auto* qp = static_cast<const uint8_t*>(q);
-  auto* ap = static_cast<const uint16_t*>(alpha);
-  auto* zp = static_cast<const uint8_t*>(zero_points);
-  auto* pp = static_cast<uint8_t*>(packets);
   const bool g64 = group_size == 64;
   if (format == PacketFormat::kNativeSym) {
-    if (g64) hipLaunchKernelGGL((pack_native_kernel<64, PacketFormat::kNativeSym>), grid, dim3(kTileCols), 0, stream, qp, ap, zp, pp, k, ng);
-    else hipLaunchKernelGGL((pack_native_kernel<128, PacketFormat::kNativeSym>), grid, dim3(kTileCols), 0, stream, qp, ap, zp, pp, k, ng);
-  } else if (format == PacketFormat::kNativeAsym) {
-    if (g64) hipLaunchKernelGGL((pack_native_kernel<64, PacketFormat::kNativeAsym>), grid, dim3(kTileCols), 0, stream, qp, ap, zp, pp, k, ng);
-    else hipLaunchKernelGGL((pack_native_kernel<128, PacketFormat::kNativeAsym>), grid, dim3(kTileCols), 0, stream, qp, ap, zp, pp, k, ng);
-  } else {
-    return hipErrorInvalidValue;
+    return g64 ? launch_pack<64, PacketFormat::kNativeSym>(q, alpha, zero_points, packets, n, k, stream)
+               : launch_pack<128, PacketFormat::kNativeSym>(q, alpha, zero_points, packets, n, k, stream);
   }
-  return hipGetLastError();
+  if (format == PacketFormat::kNativeAsym) {
+    return g64 ? launch_pack<64, PacketFormat::kNativeAsym>(q, alpha, zero_points, packets, n, k, stream)
+               : launch_pack<128, PacketFormat::kNativeAsym>(q, alpha, zero_points, packets, n, k, stream);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_arc_to_native(const void* arc, void* native, int n, int k, int group_size,
