@@ -347,10 +347,11 @@ arc_to_native_kernel(const uint8_t* __restrict__ arc, uint8_t* __restrict__ nati
       }
     }
   }
-  if (zp < 0) {
-    __hip_atomic_fetch_or(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    zp = 0;
+  // *bad is host memory: one store a wave, and none for packets that convert
+  if (__any(zp < 0) && (c & 63) == 0) {
+    __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+  zp = max(zp, 0);
   if constexpr (F == PacketFormat::kNativeAsym) {
     store_neg_zp<G>(s, static_cast<uint32_t>(zp));
   }

@@ -21,9 +21,15 @@ Differences from the reference, by design:
 from __future__ import annotations
 
 import os
+from functools import lru_cache
 from typing import TYPE_CHECKING, Any
 
 from fast_kernels.native import native_build_info, native_module
+
+try:
+    import torch as _torch
+except ImportError:  # pragma: no cover - every op then raises RuntimeError
+    _torch = None
 
 if TYPE_CHECKING:  # pragma: no cover
     import torch
@@ -61,11 +67,9 @@ LAYOUT_TO_GROUP_SIZE: dict[str, int] = {
 
 
 def _require_torch() -> Any:
-    try:
-        import torch
-    except ImportError as exc:  # pragma: no cover
-        raise RuntimeError("PyTorch is required for decode_quant_linear ops") from exc
-    return torch
+    if _torch is None:  # pragma: no cover
+        raise RuntimeError("PyTorch is required for decode_quant_linear ops")
+    return _torch
 
 
 def hip_decode_available() -> bool:
@@ -92,6 +96,7 @@ def arc_packet_stride_bytes(group_size: int) -> int:
     return (128 * (group_size // 2)) + (2 * 128 * 2)
 
 
+@lru_cache(maxsize=1)
 def _require_gpu_backend() -> Any:
     native = native_module()
     if not hip_decode_available():
@@ -106,7 +111,7 @@ def _check_gpu_tensor(tensor: Any, *, name: str, dtype: Any, ndim: int) -> None:
     dtypes = dtype if isinstance(dtype, tuple) else (dtype,)
     if tensor.dtype not in dtypes:
         raise TypeError(f"{name} must have dtype {' or '.join(str(d) for d in dtypes)}")
-    if tensor.ndim != ndim:
+    if tensor.dim() != ndim:
         raise ValueError(f"{name} must be {ndim}D")
     if not tensor.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor")
@@ -115,16 +120,23 @@ def _check_gpu_tensor(tensor: Any, *, name: str, dtype: Any, ndim: int) -> None:
 
 
 def _check_same_device(*named_tensors: tuple[str, Any]) -> None:
-    devices = {tensor.device for _, tensor in named_tensors}
-    if len(devices) <= 1:
+    first = named_tensors[0][1].get_device()
+    for _, tensor in named_tensors:
+        if tensor.get_device() != first:
+            break
+    else:
         return
     summary = ", ".join(f"{name}={tensor.device}" for name, tensor in named_tensors)
     raise ValueError(f"all GPU tensors must be on the same device: {summary}")
 
 
 def _current_stream_ptr(device: Any) -> int:
+    """Raw handle of the device's current stream, without a torch.cuda.Stream object (4 us)."""
     torch = _require_torch()
-    return int(torch.cuda.current_stream(device=device).cuda_stream)
+    index = device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _device_index(device: Any) -> int:
@@ -212,15 +224,29 @@ def arc_workspace(device: Any, nbytes: int) -> Any:
     return ws
 
 
-def _plan_workspace(plan: dict[str, int], device: Any) -> tuple[Any, int, int]:
-    """(tensor to keep until the launch, pointer, bytes) of a plan's workspace. A row-tile plan's
+@lru_cache(maxsize=1024)
+def _workspace_plan(device: int, kind: str, *shape: Any) -> tuple[int, int]:
+    """(workspace bytes, schedule) of a launch, by its shape: a plan depends on nothing else."""
+    native = _require_gpu_backend()
+    if kind == "plain":
+        plan = native.arc_w4a16_plan(*shape)
+    elif kind == "fused":
+        plan = native.w4a16_plan_fused(*shape)
+    else:
+        plan = native.w4a16_plan_rmsnorm(*shape)
+    return int(plan["workspace_bytes"]), int(plan["schedule"])
+
+
+def _plan_workspace(device: Any, kind: str, *shape: Any) -> tuple[Any, int, int]:
+    """(tensor to keep until the launch, pointer, bytes) of a launch's workspace. A row-tile plan's
     (prepared activations, partial tiles) grows with the rows and needs no zeros: it is the
     allocator's, for this call. The others' counters are kept per stream (arc_workspace)."""
-    nbytes = int(plan["workspace_bytes"])
+    torch = _require_torch()
+    nbytes, schedule = _workspace_plan(torch.cuda.current_device(), kind, *shape)
     if nbytes == 0:
         return None, 0, 0
-    if plan["schedule"] == SCHEDULE_TILES:
-        ws = _require_torch().empty(nbytes, device=device, dtype=_require_torch().uint8)
+    if schedule == SCHEDULE_TILES:
+        ws = torch.empty(nbytes, device=device, dtype=torch.uint8)
     else:
         ws = arc_workspace(device, nbytes)
     return ws, ws.data_ptr(), ws.numel()
@@ -444,8 +470,9 @@ def arc_w4a16_forward(
     act = _act_code(out_dtype)
     requested = 0 if split_k_slices is None else split_k_slices
     kernel = _IMPL_KERNEL[resolved]
-    plan = native.arc_w4a16_plan(batch, n, k, group_size, act, requested, 0, 0, kernel)
-    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+    _ws, ws_ptr, ws_bytes = _plan_workspace(
+        activations.device, "plain", batch, n, k, group_size, act, requested, 0, 0, kernel
+    )
     if kernel != KERNEL_AUTO:
         native.w4a16_forward_kernel(
             activations.data_ptr(), packets.data_ptr(), output.data_ptr(), ws_ptr, ws_bytes,

@@ -237,8 +237,9 @@ def arc_w4a16_forward_native(
         raise ValueError("split_k_slices must be positive")
     requested = 0 if split_k_slices is None else int(split_k_slices)
     act = _act_code(activations.dtype)
-    plan = native.arc_w4a16_plan(batch, n, k, group_size, act, requested, 0, code)
-    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+    _ws, ws_ptr, ws_bytes = _plan_workspace(
+        activations.device, "plain", batch, n, k, group_size, act, requested, 0, code
+    )
     native.arc_w4a16_forward_native(
         activations.data_ptr(), packets.data_ptr(), output.data_ptr(), ws_ptr, ws_bytes, batch,
         n, k, group_size, code, act, requested, _current_stream_ptr(activations.device),
@@ -290,16 +291,18 @@ def arc_w4a16_forward_rmsnorm(
     requested = 0 if split_k_slices is None else int(split_k_slices)
     act = _act_code(activations.dtype)
     if requested == 0:
-        plan = native.w4a16_plan_fused(batch, n, k, group_size, act, 0, code, False)
-        _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+        _ws, ws_ptr, ws_bytes = _plan_workspace(
+            activations.device, "fused", batch, n, k, group_size, act, 0, code, False
+        )
         native.w4a16_forward_fused(
             activations.data_ptr(), norm_weight.data_ptr(), float(eps), packets.data_ptr(),
             output.data_ptr(), ws_ptr, ws_bytes, batch, n, k, group_size, code, act, False,
             _current_stream_ptr(activations.device),
         )
         return output
-    plan = native.w4a16_plan_rmsnorm(batch, n, k, group_size, act, requested, 0, code)
-    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+    _ws, ws_ptr, ws_bytes = _plan_workspace(
+        activations.device, "rmsnorm", batch, n, k, group_size, act, requested, 0, code
+    )
     native.w4a16_forward_rmsnorm(
         activations.data_ptr(), norm_weight.data_ptr(), float(eps), packets.data_ptr(),
         output.data_ptr(), ws_ptr, ws_bytes, batch, n, k, group_size, code, act, requested,
@@ -355,8 +358,9 @@ def arc_w4a16_forward_silu_mul(
         _check_same_device(("activations", activations), ("norm_weight", norm_weight))
         norm_ptr = norm_weight.data_ptr()
     act = _act_code(activations.dtype)
-    plan = native.w4a16_plan_fused(batch, n, k, group_size, act, 0, code, True)
-    _ws, ws_ptr, ws_bytes = _plan_workspace(plan, activations.device)
+    _ws, ws_ptr, ws_bytes = _plan_workspace(
+        activations.device, "fused", batch, n, k, group_size, act, 0, code, True
+    )
     native.w4a16_forward_fused(
         activations.data_ptr(), norm_ptr, float(eps), packets.data_ptr(), output.data_ptr(),
         ws_ptr, ws_bytes, batch, n, k, group_size, code, act, True,
