@@ -22,6 +22,8 @@ constexpr int kTileWaveK = 256;
 
 struct TileShape {
   int rows = 0;         // activation rows of the launch
+  double us = 0;        // estimated time on MI355X
+  bool direct = false;  // the workgroups stage x themselves: no prepare launch, no fused neighbour
   int bm = 0, bn = 0;   // rows and columns of a workgroup's tile
   int mtiles = 0, col_tiles = 0;
   int unit_groups = 0;  // groups of a unit, the grain of the K splits
@@ -48,8 +50,8 @@ struct TileLaunch {
 };
 
 // Work split and workspace for `rows` (at most kTileMaxRows) on cu_count CUs; the workspace starts
-// with counter_bytes of counters.
-TileShape tile_shape(int rows, int n, int k, int group_size, bool silu, int cu_count,
+// with counter_bytes of counters. direct: at most 32 rows.
+TileShape tile_shape(int rows, int n, int k, int group_size, bool direct, int cu_count,
                      size_t counter_bytes);
 
 hipError_t launch_w4a16_gemm_tile(const TileLaunch& l, const TileShape& s, hipStream_t stream);

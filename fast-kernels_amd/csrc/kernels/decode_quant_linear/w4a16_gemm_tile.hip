@@ -1,11 +1,13 @@
 // W4A16 GEMM over row tiles on the gfx950 matrix cores: 17 activation rows and more (batched
 // serving, chunks of a prompt), over reference packets or native slabs.
 //
-// A first launch (tile_prepare_kernel) writes the activations in the order the tiles read them:
+// Above 32 rows, and under a fused neighbour, a first launch (tile_prepare_kernel) writes the activations in the order the tiles read them:
 // re-paired (x0,x4)(x1,x5)(x2,x6)(x3,x7) like the code words unpack, [32-row block][group][16-byte
 // unit][row], so staging is a straight copy and every LDS access is 512 consecutive bytes per
 // half wave; beside them the (row, group) sums. It applies the RMSNorm where one is fused, so
-// that costs no pass of its own.
+// that costs no pass of its own. Up to 32 plain rows the tiles stage the activations themselves: the
+// launch costs 4-5 us there and the pairing little (32 rows, bf16 native: 28672 x 4096 23.6 -> 22.1
+// us, 4096 x 14336 18.9 -> 16.0, 10240 x 8192 21.1 -> 18.1, 4096 x 4096 12.9 -> 11.0).
 //
 // The GEMM's workgroup (8 waves) owns BM rows x BN columns. Each wave owns whole 32-column slices
 // of the tile, reads their code words straight into registers (each word is unpacked once per
@@ -184,13 +186,14 @@ __global__ void __launch_bounds__(kPrepThreads) tile_prepare_kernel(PrepareParam
 }
 
 struct TileParams {
+  const uint16_t* x;  // kDirect: the activations [M, K]
   const u32x4_t* xs;
   const u32x4_t* sums;
   const uint8_t* packets;
   uint16_t* out;
   float* partials;
   uint32_t* counters;
-  int M, N, NG, mtiles, tile_units, per, splits;
+  int M, N, K, NG, mtiles, tile_units, per, splits;
   int grid, xcd_remap;
   int vector_out;  // out rows are 16-byte aligned
 };
@@ -352,14 +355,16 @@ __device__ __forceinline__ uint32_t silu_mul_pair(uint32_t gw, uint32_t uw) {
 // One output in plain fp32 arithmetic on activations 2^-64 times smaller: for bf16 outputs that
 // came out infinite or NaN. The tile's accumulators hold sums of (128 + q) x, which overflow from
 // |x| of about 2^113; the result itself may still be finite.
-template <int G, PacketFormat F>
+template <int G, PacketFormat F, bool kDirect>
 __device__ __forceinline__ uint16_t plain_bf16_output(const TileParams& p, int row, int col) {
   constexpr int WR = G / 8;
   constexpr int kStride = format_packet_stride(G, F);
   const uint8_t* base =
       p.packets + static_cast<size_t>(is_native(F) ? col / kSliceCols : col / kTileCols) * p.NG * kStride;
   const int c = is_native(F) ? col % kSliceCols : col % kTileCols;
-  const u32x4_t* xr = p.xs + static_cast<size_t>(row / kBlockRows) * p.NG * (WR * kBlockRows) + row % kBlockRows;
+  const u32x4_t* xr =
+      kDirect ? reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(row) * p.K)
+              : p.xs + static_cast<size_t>(row / kBlockRows) * p.NG * (WR * kBlockRows) + row % kBlockRows;
   float y = 0.0f;
 #pragma unroll 1
   for (int g = 0; g < p.NG; ++g) {
@@ -368,13 +373,20 @@ __device__ __forceinline__ uint16_t plain_bf16_output(const TileParams& p, int r
     float sum = 0.0f;
 #pragma unroll 1
     for (int w = 0; w < WR; ++w) {
-      const u32x4_t x = xr[(g * WR + window_slot<G>(w, is_native(F))) * kBlockRows];
+      u32x4_t x;  // paired: values i and i + 4
+      if constexpr (kDirect) {
+        const u32x4_t v = xr[g * WR + w];
+        const uint4 q = pair_activations(make_uint4(v.x, v.y, v.z, v.w));
+        x = u32x4_t{q.x, q.y, q.z, q.w};
+      } else {
+        x = xr[(g * WR + window_slot<G>(w, is_native(F))) * kBlockRows];
+      }
       constexpr int U = native_unit_words(G);
       const int at = is_native(F) ? native_word_offset(G, c / 16, w / U, c % 16, w % U)
                                   : (w * kTileCols + c) * 4;
       const uint32_t word = *reinterpret_cast<const uint32_t*>(group + at);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {  // paired: values i and i + 4
+      for (int i = 0; i < 4; ++i) {
         const float lo = bf16_bits_to_float(static_cast<uint16_t>(x[i])) * 0x1p-64f;
         const float hi = bf16_bits_to_float(static_cast<uint16_t>(x[i] >> 16)) * 0x1p-64f;
         dot = fmaf(static_cast<float>((word >> (4 * i)) & 15u), lo, dot);
@@ -408,7 +420,11 @@ __device__ __forceinline__ bool has_non_finite_bf16(uint32_t pair) {
   return (pair & 0x7f80u) == 0x7f80u || (pair & 0x7f800000u) == 0x7f800000u;
 }
 
-template <class T, Act A, PacketFormat F, bool kSilu, bool kOnce>
+// kDirect: the workgroup stages the activations itself, from x, instead of copying prepared ones: a
+// wave reads a row's 512 values of the chunk, pairs them and adds up the groups' sums, a row per
+// window between the MFMAs. LDS rows are swizzled by the unit's place (consecutive lanes store
+// consecutive units of one row, 512 bytes apart).
+template <class T, Act A, PacketFormat F, bool kSilu, bool kOnce, bool kDirect>
 __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p) {
   constexpr int G = T::G;
   constexpr int RS = T::RS;
@@ -504,16 +520,90 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
     // by every thread, more than once where there are fewer units: no branch in the loop
     buf[T::kXUnits + tid % T::kSUnits] = sreg;
   };
+  // kDirect: lane l takes unit l of the chunk's 64 units of a row (a chunk of four wave groups is
+  // 512 values), the wave rows wave, wave + 8, ... of the tile; rows and units past the end repeat
+  // the last one.
+  constexpr int WR = G / 8;
+  static_assert(!kDirect || (T::WP == 4 && T::kXPer == T::kBM / kTileWaves), "a row per wave and pass");
+  const int d_slot = window_slot<G>(lane % WR, is_native(F));
+  const uint32_t d_store = static_cast<uint32_t>(
+      (lane / WR * T::kBlocks * WR + d_slot) * kBlockRows + (wave ^ (d_slot & 7)));
+  float d_sum = 0.0f;  // of the row of pass lane % kXPer
+  auto direct_load = [&](int g0, int it) {
+    const int row = min(mt * T::kBM + it * kTileWaves + wave, p.M - 1);
+    const uint32_t unit = static_cast<uint32_t>(min(g0 * WR + lane, p.NG * WR - 1));
+    xreg[it] = reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(row) * p.K)[unit];
+  };
+  auto direct_store = [&](u32x4_t* buf, int it) {
+    const u32x4_t v = xreg[it];
+    const uint4 xp = pair_activations(make_uint4(v.x, v.y, v.z, v.w));
+    float s = 0.0f;
+    if constexpr (A == Act::kF16) {
+      constexpr uint32_t kOnes = 0x3c003c00u;
+      s = dot2<A>(xp.w, kOnes, dot2<A>(xp.z, kOnes, dot2<A>(xp.y, kOnes, dot2<A>(xp.x, kOnes, s))));
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        s += bf16_bits_to_float(static_cast<uint16_t>(v[q])) +
+             __builtin_bit_cast(float, v[q] & 0xffff0000u);
+      }
+    }
+    s = group_sum<WR>(s);
+    d_sum = lane % T::kXPer == it ? s : d_sum;
+    const int row8 = it * kTileWaves;  // of the pass; the wave's row is row8 + wave
+    buf[d_store + (row8 / kBlockRows * WR * kBlockRows + row8 % kBlockRows)] =
+        u32x4_t{xp.x, xp.y, xp.z, xp.w};
+  };
+  // The sums of the wave's rows, one (row, group) a lane: lane % kXPer is the pass (lanes that
+  // share one write the same values).
+  auto direct_sums = [&](u32x4_t* buf) {
+    const int it = lane % T::kXPer;
+    uint32_t q[3];
+    bf16_parts(d_sum, q);
+    const int row = it * kTileWaves + wave;
+    buf[T::kXUnits + (lane / WR * T::kBlocks + row / kBlockRows) * kBlockRows + row % kBlockRows] =
+        u32x4_t{q[0] | (q[0] << 16), q[0] | (q[1] << 16), q[1] | (q[1] << 16), q[2] | (q[2] << 16)};
+  };
+  auto stage_load_all = [&](int g0) {
+    if constexpr (kDirect) {
+#pragma unroll
+      for (int it = 0; it < T::kXPer; ++it) {
+        direct_load(g0, it);
+      }
+    } else {
+      stage_load(g0);
+    }
+  };
+  auto stage_store_all = [&](u32x4_t* buf) {
+    if constexpr (kDirect) {
+#pragma unroll
+      for (int it = 0; it < T::kXPer; ++it) {
+        direct_store(buf, it);
+      }
+      direct_sums(buf);
+    } else {
+      stage_store(buf);
+    }
+  };
 
   float16_t y[RS][CS] = {};
-  stage_load(u_begin * T::kUnitGroups);
+  stage_load_all(u_begin * T::kUnitGroups);
   load_weights(u_begin * T::kUnitGroups, wreg[0]);
-  stage_store(lds);
-  stage_load(u_begin * T::kUnitGroups + T::kChunkGroups);
+  stage_store_all(lds);
+  stage_load_all(u_begin * T::kUnitGroups + T::kChunkGroups);
   load_weights(u_begin * T::kUnitGroups + T::kChunkGroups, wreg[1]);
   __syncthreads();
   const u32x4_t* x_lane = lds + wp * KG * (T::kBlocks * T::kGroupUnits) +
-                          wr * RS * T::kGroupUnits + lane;
+                          wr * RS * T::kGroupUnits + (kDirect ? 0 : lane);
+  // kDirect: a window's place in LDS is 64 units, half h's 32 rows second, the row swizzled by the
+  // place, which repeats every four windows.
+  uint32_t x_swizzled[4];
+  if constexpr (kDirect) {
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+      x_swizzled[z] = half * kBlockRows + ((lane & 31) ^ (2 * z + half));
+    }
+  }
   const u32x4_t* s_lane = lds + T::kXUnits + (wp * KG * T::kBlocks + wr * RS) * kBlockRows + (lane & 31);
   for (int u = u_begin; u < u_end; ++u) {
     // Past the last unit the loads read group 0, which is in the L2.
@@ -525,8 +615,11 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
       // The next chunk's activations, loaded a chunk ago, into the other buffer; then the loads of
       // the chunk after it. All loads are unconditional: a branch around them would make the
       // compiler wait for every load in flight where the paths join.
-      stage_store(lds + (h ^ 1) * T::kBufUnits);
-      stage_load(g_next + h * T::kChunkGroups);
+      u32x4_t* other = lds + (h ^ 1) * T::kBufUnits;
+      if constexpr (!kDirect) {
+        stage_store(other);
+        stage_load(g_next + h * T::kChunkGroups);
+      }
       const u32x4_t* xg = x_lane + h * T::kBufUnits;
       const u32x4_t* sg = s_lane + h * T::kBufUnits;
       const int g_wave = u * T::kUnitGroups + h * T::kChunkGroups + wp * KG;
@@ -538,7 +631,11 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
         const int off = (w / T::kWindows) * (T::kBlocks * T::kGroupUnits) + w % T::kWindows * 64;
 #pragma unroll
         for (int i = 0; i < RS; ++i) {
-          a[w % (kAhead + 1)][i] = xg[off + i * T::kGroupUnits];
+          if constexpr (kDirect) {
+            a[w % (kAhead + 1)][i] = (xg + x_swizzled[w % 4])[off + i * T::kGroupUnits];
+          } else {
+            a[w % (kAhead + 1)][i] = xg[off + i * T::kGroupUnits];
+          }
         }
       };
 #pragma unroll
@@ -577,6 +674,15 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
 #pragma unroll
           for (int i = 0; i < RS; ++i) {
             d[i][j] = mfma<A>(a[w % (kAhead + 1)][i], q, d[i][j]);
+          }
+        }
+        if constexpr (kDirect) {
+          if (w < T::kXPer) {
+            direct_store(other, w);
+            direct_load(g_next + h * T::kChunkGroups, w);
+          }
+          if (w == T::kXPer - 1) {
+            direct_sums(other);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -741,7 +847,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
           for (int q = 0; q < 8; ++q) {
             uint16_t* at = tile16 + row * T::kOutPitch + tile_col + q;
             if ((*at & 0x7f80u) == 0x7f80u) {
-              *at = plain_bf16_output<G, F>(p, row0 + row, col + q);
+              *at = plain_bf16_output<G, F, kDirect>(p, row0 + row, col + q);
             }
           }
           o = *reinterpret_cast<const u32x4_t*>(tile16 + row * T::kOutPitch + tile_col);
@@ -777,9 +883,9 @@ using Tile64 = Tile<G, 2, 2, 1, 2, 4>;   // 64 x 128
 template <int G>
 using Tile128 = Tile<G, 2, 2, 2, 4, 1>;  // 128 x 256
 
-template <class T, Act A, PacketFormat F, bool kSilu, bool kOnce>
+template <class T, Act A, PacketFormat F, bool kSilu, bool kOnce, bool kDirect = false>
 hipError_t launch_tile(const TileParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((tile_gemm_kernel<T, A, F, kSilu, kOnce>), dim3(p.grid), dim3(kTileThreads),
+  hipLaunchKernelGGL((tile_gemm_kernel<T, A, F, kSilu, kOnce, kDirect>), dim3(p.grid), dim3(kTileThreads),
                      T::kLdsBytes, stream, p);
   return hipGetLastError();
 }
@@ -787,16 +893,39 @@ hipError_t launch_tile(const TileParams& p, hipStream_t stream) {
 template <int G, Act A, PacketFormat F>
 hipError_t launch_typed(const TileLaunch& l, const TileShape& s, hipStream_t stream) {
   char* ws = static_cast<char*>(l.workspace);
+  TileParams p;
+  p.x = static_cast<const uint16_t*>(l.x);
+  p.xs = reinterpret_cast<const u32x4_t*>(ws + s.xs);
+  p.sums = reinterpret_cast<const u32x4_t*>(ws + s.sums);
+  p.packets = static_cast<const uint8_t*>(l.packets);
+  p.out = static_cast<uint16_t*>(l.out);
+  p.partials = reinterpret_cast<float*>(ws + s.partials);
+  p.counters = reinterpret_cast<uint32_t*>(ws);
+  p.M = l.M;
+  p.N = l.N;
+  p.K = l.K;
+  p.NG = l.K / G;
+  p.mtiles = s.mtiles;
+  p.tile_units = s.units;
+  p.per = s.per;
+  p.splits = s.splits;
+  p.grid = s.grid;
+  p.xcd_remap = s.grid % 8 == 0 ? s.grid / 8 : 0;
+  p.vector_out = reinterpret_cast<uintptr_t>(l.out) % 16 == 0;
+  if (s.direct) {
+    return s.bm == 32 ? launch_tile<Tile32<G>, A, F, false, true, true>(p, stream)
+                      : hipErrorInvalidValue;
+  }
   PrepareParams q;
-  q.x = static_cast<const uint16_t*>(l.x);
+  q.x = p.x;
   q.gamma = static_cast<const uint16_t*>(l.norm_weight);
   q.xs = reinterpret_cast<uint4*>(ws + s.xs);
   q.sums = reinterpret_cast<uint4*>(ws + s.sums);
-  q.counters = reinterpret_cast<uint32_t*>(ws);
+  q.counters = p.counters;
   q.n_counters = s.splits > 1 ? s.mtiles * s.col_tiles : 0;
   q.M = l.M;
   q.K = l.K;
-  q.NG = l.K / G;
+  q.NG = p.NG;
   q.eps = l.eps;
   q.quarters = is_native(F);
   const dim3 pgrid(static_cast<unsigned int>(s.mtiles * s.bm / kPrepRows),
@@ -809,23 +938,6 @@ hipError_t launch_typed(const TileLaunch& l, const TileShape& s, hipStream_t str
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) {
     return e;
   }
-  TileParams p;
-  p.xs = reinterpret_cast<const u32x4_t*>(q.xs);
-  p.sums = reinterpret_cast<const u32x4_t*>(q.sums);
-  p.packets = static_cast<const uint8_t*>(l.packets);
-  p.out = static_cast<uint16_t*>(l.out);
-  p.partials = reinterpret_cast<float*>(ws + s.partials);
-  p.counters = q.counters;
-  p.M = l.M;
-  p.N = l.N;
-  p.NG = q.NG;
-  p.mtiles = s.mtiles;
-  p.tile_units = s.units;
-  p.per = s.per;
-  p.splits = s.splits;
-  p.grid = s.grid;
-  p.xcd_remap = s.grid % 8 == 0 ? s.grid / 8 : 0;
-  p.vector_out = reinterpret_cast<uintptr_t>(l.out) % 16 == 0;
   constexpr bool kCanSilu = is_native(F);
   if (l.silu) {
     if constexpr (kCanSilu) {
@@ -858,28 +970,34 @@ hipError_t launch_format(const TileLaunch& l, const TileShape& s, hipStream_t st
 
 }  // namespace
 
-// Tile choice and K splits by a cost model of the launch, in us, fitted to timestamps of the kernel's
-// phases on MI355X: workgroups run one per CU, in rounds of start-up (first loads), units, end
-// (wave groups' sums, output) and, with K split, the fix-up (partials out, counter, partials in).
+// Tile choice and K splits by a cost model of the launch, in us, fitted to 560 measured launches (17
+// to 512 rows, 512 to 16384 columns, K from 512 to 6144, bf16 native slabs, MI355X; the fit's
+// standard deviation is 4-8 %): workgroups run one per CU, in rounds of start-up and end (first
+// loads; wave groups' sums, output), units and, with K split, the fix-up (partials out, counter,
+// partials in); `prepare` is the launch before them.
 struct TileCost {
   int bm, bn, phases;
-  double unit, fixed, fix, fix_per_split;
+  double unit, fixed, fix, fix_per_split, prepare;
 };
-constexpr TileCost kTileCosts[] = {
-    {32, 128, 4, 3.2, 4.5, 3.5, 0.2},
-    {64, 128, 4, 4.8, 5.5, 4.0, 0.3},
-    {128, 256, 1, 4.0, 6.0, 4.0, 2.0},
+constexpr TileCost kTileCosts64[] = {
+    {32, 128, 4, 4.1, 4.5, 3.0, 0.1, 2.0},
+    {64, 128, 4, 6.5, 6.4, 1.9, 0.8, 1.9},
+    {128, 256, 1, 4.55, 6.1, 2.5, 2.8, 4.6},
+};
+constexpr TileCost kTileCosts128[] = {
+    {32, 128, 4, 3.4, 4.1, 2.8, 0.1, 2.0},
+    {64, 128, 4, 5.8, 6.0, 1.8, 0.85, 1.7},
+    {128, 256, 1, 3.8, 7.25, 2.0, 3.1, 2.8},
 };
 constexpr int kMaxTileSplits = 16;
 
-TileShape tile_shape(int rows, int n, int k, int group_size, bool silu, int cu_count,
+TileShape tile_shape(int rows, int n, int k, int group_size, bool direct, int cu_count,
                      size_t counter_bytes) {
-  (void)silu;
   TileShape s;
+  s.direct = direct;
   s.rows = rows;
   const int ng = k / group_size;
-  double best = 0;
-  for (const TileCost& c : kTileCosts) {
+  for (const TileCost& c : group_size == 64 ? kTileCosts64 : kTileCosts128) {
     // the smallest tile serves rows that fit it, the largest more rows than the next one's
     if ((c.bm == 32 && rows > 32) || (c.bm == 64 && rows <= 32) || (c.bm == 128 && rows <= 64)) {
       continue;
@@ -896,9 +1014,10 @@ TileShape tile_shape(int rows, int n, int k, int group_size, bool silu, int cu_c
       const long long tiles = static_cast<long long>(mtiles) * col_tiles;
       const long long rounds = (tiles * splits + cu_count - 1) / cu_count;
       const double fix = splits > 1 ? c.fix + c.fix_per_split * splits : 0.0;
-      const double cost = static_cast<double>(rounds) * (per * c.unit + c.fixed + fix);
-      if (s.bm == 0 || cost < best) {
-        best = cost;
+      const double cost = static_cast<double>(rounds) * (per * c.unit + c.fixed + fix) +
+                          (direct ? 0.0 : c.prepare);
+      if (s.bm == 0 || cost < s.us) {
+        s.us = cost;
         s.bm = c.bm;
         s.bn = c.bn;
         s.mtiles = mtiles;
@@ -914,16 +1033,18 @@ TileShape tile_shape(int rows, int n, int k, int group_size, bool silu, int cu_c
   auto align = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t padded = static_cast<size_t>(s.mtiles) * s.bm;
   s.partials = counter_bytes;
-  s.sums = align(s.partials + (s.splits > 1 ? static_cast<size_t>(s.grid) * s.bm *
+  const size_t partials_end = align(s.partials + (s.splits > 1 ? static_cast<size_t>(s.grid) * s.bm *
                                                              s.bn * sizeof(float)
                                                        : 0));
+  s.sums = partials_end;
   s.xs = align(s.sums + padded * ng * 16);
-  s.end = s.xs + padded * k * 2;
+  s.end = direct ? (s.splits > 1 ? partials_end : 0) : s.xs + padded * k * 2;
   return s;
 }
 
 hipError_t launch_w4a16_gemm_tile(const TileLaunch& l, const TileShape& s, hipStream_t stream) {
-  if (l.M != s.rows || (l.silu && l.N % 256 != 0)) {
+  if (l.M != s.rows || (l.silu && l.N % 256 != 0) ||
+      (s.direct && (l.silu || l.norm_weight != nullptr || s.mtiles != 1))) {
     return hipErrorInvalidValue;
   }
   switch (l.format) {

@@ -94,8 +94,15 @@ struct ArcW4A16Plan {
 // each workgroup streaming one contiguous range of slabs across slices with the whole activation
 // row staged in LDS (w4a16_gemv_stream.hip).
 // kScheduleTiles: 17 rows and more on the row-tile GEMM (w4a16_gemm_tile.hip): m_tile x slice_cols
-// tiles, K in max_tile_contributors splits.
-enum Schedule : int { kScheduleRuns = 0, kSchedulePairs = 1, kScheduleStream = 2, kScheduleTiles = 3 };
+// tiles, K in max_tile_contributors splits; kScheduleTilesDirect: the same with the activations staged
+// by the tiles, without a launch that prepares them.
+enum Schedule : int {
+  kScheduleRuns = 0,
+  kSchedulePairs = 1,
+  kScheduleStream = 2,
+  kScheduleTiles = 3,
+  kScheduleTilesDirect = 4,
+};
 
 // The launch the GEMV will use for this shape on the current device. split_k_slices = 0 picks
 // the built-in policy; S > 0 gives every workgroup ceil(K / G / S) groups of whole 128-column

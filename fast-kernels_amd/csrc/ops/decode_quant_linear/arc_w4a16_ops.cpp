@@ -14,6 +14,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstdlib>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -153,9 +154,22 @@ constexpr int kMaxSlicesPerTile = 4;
 // Longest K for which one-row native plans stream slice pairs.
 constexpr int kMaxPairK = 4096;
 // Fewest rows the row-tile GEMM takes from the automatic dispatch: what the 2-16-row kernels, which
-// read the weights once for up to 16 rows, do not take (measured over 16 drawn shapes of 17-768
-// rows: 1.16-2.4 times faster than 16-row tiles).
+// read the weights once for up to 16 rows, do not take. Among those the 16-row tiles keep the calls
+// they are estimated to be faster at: few columns and little K, where a launch is mostly start-up and
+// the chip has room for a workgroup per 16 rows (16-row and row tiles, 64 rows, bf16, G128: 2048 x
+// 1024 8.1 and 12.9 us, 4864 x 4096 19.6 and 18.5, 16384 x 4096 34.6 and 24.4).
 constexpr int kTileMinBatch = 17;
+// Most rows whose activations the tiles stage themselves: the 32-row tile's, where the launch that
+// prepares them costs more than every workgroup pairing its own (32 rows, bf16, native_sym, prepared
+// and direct: 4096x4096 12.9 and 11.0 us, 4096x14336 18.9 and 16.0, 28672x4096 23.6 and 22.1). The
+// 64-row tile has no registers left for it (64 rows: 10240x8192 27.1 and 30.8, 28672x4096 27.6 and
+// 34.6).
+constexpr int kTileDirectMaxRows = 32;
+// The row tiles' estimate has to be this part of the other kernel's: the estimates' errors are about
+// 7 % each. Over the 560 shapes they were fitted to, the choice costs 0.3 % against the faster of
+// the two at every shape.
+constexpr double kTileMargin = 0.92;
+bool tile_direct(int batch, bool plain) { return plain && batch <= kTileDirectMaxRows; }
 
 // Grid, run length and fix-up workspace of a stream-K plan over tiles x slices x num_groups units.
 void finish_plan(ArcW4A16Plan& plan, long long tiles, long long slices, int num_groups,
@@ -228,8 +242,12 @@ bool arc_quarter_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_siz
                       int split_k_slices, int cu_count, bool cu_count_given);
 bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size,
                           int split_k_slices, int cu_count, bool cu_count_given);
-bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool silu,
-               int cu_count);
+bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
+               int cu_count, double other_us);
+double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count);
+bool is_tile_schedule(int schedule) {
+  return schedule == kScheduleTiles || schedule == kScheduleTilesDirect;
+}
 
 }  // namespace
 
@@ -239,7 +257,8 @@ ArcW4A16Plan plan_arc_w4a16_for_cu_count(int batch, int n, int k, int group_size
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, fk::gemv_m_tile_for_batch(batch));
   if (split_k_slices == 0 && batch >= kTileMinBatch &&
-      tile_plan(plan, batch, n, k, group_size, false, cu_count)) {
+      tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
+                row16_us(plan, group_size, cu_count))) {
     return plan;
   }
   if (!arc_mfma_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true) &&
@@ -368,10 +387,29 @@ bool fused_mfma_takes_small(int batch, bool silu) {
 // RMSNorm + 8192 x 11008 G64 + SiLU 34 / 54 / 94 against 26.8, 1024 x 2048 at 8-16 rows 12.0
 // against 13.1, 2048 x 4096 G64 at 8 rows 15.9 against 15.2.
 long long tile_fused_min_weights(int batch) {
-  return batch >= 17 ? 0 : batch >= 5 ? 4LL << 20 : batch >= 3 ? 32LL << 20 : 84LL << 20;
+  return batch >= 5 ? 4LL << 20 : batch >= 3 ? 32LL << 20 : 84LL << 20;
 }
-bool tile_takes_fused(int batch, int n, int k) {
-  return batch >= 2 && static_cast<long long>(n) * k >= tile_fused_min_weights(batch);
+// What a fused neighbour takes on the dot2 kernels, in us, for tile_plan. From 17 rows: rounds of
+// workgroups of 8 rows and one slice (SiLU: a pair of slices) over all of K, one (G128) or two (G64)
+// per CU. Measured for a round at K 768 / 2048 / 4096, bf16: RMSNorm G128 9.5 / 12.0 / 20, G64 8.4 /
+// 13.3 / 16-21 and 1.3 times that with two workgroups per CU; with SiLU G128 12.2 / 16.3 / 34, G64
+// 10.8 / 20.7 / 37. One round of little K is faster than the row tiles (40 rows, G128: 512 x 1024 9.9
+// and 13.6), two are not (2048 x 1024 18.7 and 14.1).
+double fused_dot2_us(int batch, int n, int k, int group_size, bool silu, int cu_count) {
+  if (batch < kTileMinBatch) {
+    const bool tiles =
+        batch >= 2 && static_cast<long long>(n) * k >= tile_fused_min_weights(batch);
+    return tiles ? std::numeric_limits<double>::infinity() : 0.0;
+  }
+  const double kk = k / 1024.0;
+  const long long slices = (n + fk::kSliceCols - 1) / fk::kSliceCols / (silu ? 2 : 1);
+  const long long workgroups = (batch + 7) / 8 * slices;
+  const long long resident = group_size == 64 ? 2LL * cu_count : cu_count;
+  const double rounds = static_cast<double>((workgroups + resident - 1) / resident);
+  if (group_size == 64) {
+    return rounds * (silu ? 4.8 + 7.9 * kk : (5.5 + 3.9 * kk) * (workgroups > cu_count ? 1.3 : 1.0));
+  }
+  return rounds * (silu ? 8.8 + 3.8 * kk : 7.6 + 2.3 * kk);
 }
 bool mfma_stream_enabled() {
   static const bool enabled = env_enabled("FK_W4A16_MFMA_STREAM");
@@ -832,24 +870,46 @@ bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group
          mfma_stream_plan(plan, batch, n, k, group_size, true, cu_count, cu_count_given);
 }
 
-// The row-tile GEMM (w4a16_gemm_tile.hip). More than kTileMaxRows rows run as several launches over
-// one workspace. False (plan unchanged) when the tiles outnumber the fix-up counters.
-bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool silu,
-               int cu_count) {
+// Estimated time, in us, of a plan of 16-row tiles: rounds of workgroups, each start-up and groups,
+// and the fix-up of K splits. Fitted like the row tiles' (deviation 6-8 %).
+double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
+  struct {
+    double first, per_1024_k, round, round_k, fix;
+  } const c = group_size == 64 ? decltype(c){4.4, 3.76, 1.45, 0.685, 1.9}
+                               : decltype(c){4.9, 3.88, 1.87, 0.685, 1.9};
+  const int more_rounds = (plan.workgroups + cu_count - 1) / cu_count - 1;
+  return c.first + c.round * more_rounds +
+         c.per_1024_k * plan.groups_per_workgroup * group_size / 1024 *
+             (1 + c.round_k * more_rounds) +
+         (plan.max_tile_contributors > 1 ? c.fix : 0.0);
+}
+
+// The row-tile GEMM (w4a16_gemm_tile.hip). plain: no fused neighbour; up to kTileDirectMaxRows rows
+// are then staged by the tiles themselves (kScheduleTilesDirect), without the launch that prepares
+// them. More than kTileMaxRows rows run as several launches over one workspace. False (plan
+// unchanged) when the tiles outnumber the fix-up counters, or are not estimated to be faster than
+// another kernel's other_us.
+bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
+               int cu_count, double other_us) {
+  const bool direct = tile_direct(batch, plain);
   const int rows = std::min(batch, fk::kTileMaxRows);
   const fk::TileShape s =
-      fk::tile_shape(rows, n, k, group_size, silu, cu_count, kCounterRegionBytes);
+      fk::tile_shape(rows, n, k, group_size, direct, cu_count, kCounterRegionBytes);
   std::size_t bytes = s.end;
+  double us = s.us * (batch / rows);
   if (const int rest = batch % fk::kTileMaxRows; rest != 0 && rest != rows) {
-    bytes = std::max(
-        bytes, fk::tile_shape(rest, n, k, group_size, silu, cu_count, kCounterRegionBytes).end);
+    const fk::TileShape r =
+        fk::tile_shape(rest, n, k, group_size, direct, cu_count, kCounterRegionBytes);
+    bytes = std::max(bytes, r.end);
+    us += r.us;
   }
-  if (static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters) {
+  if (static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters ||
+      us > kTileMargin * other_us) {
     return false;
   }
   plan = ArcW4A16Plan{};
   plan.m_tile = s.bm;
-  plan.schedule = kScheduleTiles;
+  plan.schedule = direct ? kScheduleTilesDirect : kScheduleTiles;
   plan.slice_cols = s.bn;
   plan.workgroups = s.grid;
   plan.groups_per_workgroup = s.per * s.unit_groups;
@@ -871,7 +931,8 @@ ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int a
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, m_tile_for_kernel(batch, kernel));
   if (plain && tiles && split_k_slices == 0 && batch >= kTileMinBatch && kernel == kKernelAuto &&
-      tile_plan(plan, batch, n, k, group_size, false, cu_count)) {
+      tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
+                row16_us(plan, group_size, cu_count))) {
     return plan;
   }
   if (plain && split_k_slices == 0 && batch >= kMfmaStreamMinBatch &&
@@ -1218,12 +1279,13 @@ void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::u
   check_hip(fk::launch_w4a16_gemv(l, stream), "w4a16_gemv launch");
 }
 
-// The launches of a kScheduleTiles plan.
+// The launches of a row-tile plan.
 void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
                std::uintptr_t output_ptr, void* workspace, int batch, int n, int k, int group_size,
                int activation_dtype, hipStream_t stream, fk::PacketFormat format, bool silu = false,
                std::uintptr_t norm_weight_ptr = 0, float eps = 0.0f) {
   const int cu_count = device_cu_count();
+  const bool direct = tile_direct(batch, !silu && norm_weight_ptr == 0);
   for (int row = 0; row < batch; row += fk::kTileMaxRows) {
     fk::TileLaunch l;
     l.M = std::min(batch - row, fk::kTileMaxRows);
@@ -1241,7 +1303,7 @@ void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
     l.norm_weight = reinterpret_cast<const void*>(norm_weight_ptr);
     l.eps = eps;
     const fk::TileShape s =
-        fk::tile_shape(l.M, n, k, group_size, silu, cu_count, kCounterRegionBytes);
+        fk::tile_shape(l.M, n, k, group_size, direct, cu_count, kCounterRegionBytes);
     check_hip(fk::launch_w4a16_gemm_tile(l, s, stream), "w4a16_gemm_tile launch");
   }
 }
@@ -1394,14 +1456,14 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
   ArcW4A16Plan plan =
       plan_arc_w4a16_for_cu_count(batch, n, k, group_size, kActivationF16, 0, device_cu_count());
-  if (plan.schedule == kScheduleTiles && !library_workspace_ready(plan.workspace_bytes, stream)) {
+  if (is_tile_schedule(plan.schedule) && !library_workspace_ready(plan.workspace_bytes, stream)) {
     // A captured call cannot allocate: the per-tile kernels need no prepared activations (and no
     // workspace at all for most shapes).
     plan = plan_for_format_impl(batch, n, k, group_size, kActivationF16, 0, device_cu_count(),
                                 kPacketArc, kKernelAuto, /*plain=*/true, /*tiles=*/false);
   }
   void* workspace = plan.workspace_bytes > 0 ? library_workspace(plan.workspace_bytes, stream) : nullptr;
-  if (plan.schedule == kScheduleTiles) {
+  if (is_tile_schedule(plan.schedule)) {
     run_tiles(activations_ptr, packets_ptr, output_ptr, workspace, batch, n, k, group_size,
               kActivationF16, stream, fk::PacketFormat::kArc);
     return;
@@ -1554,7 +1616,7 @@ void forward_with_format(std::uintptr_t activations_ptr, std::uintptr_t packets_
       plan_w4a16_for_kernel(batch, n, k, group_size, activation_dtype, split_k_slices,
                             device_cu_count(), static_cast<int>(format), kernel);
   validate_workspace(plan, workspace_ptr, workspace_bytes);
-  if (plan.schedule == kScheduleTiles) {
+  if (is_tile_schedule(plan.schedule)) {
     run_tiles(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr),
               batch, n, k, group_size, activation_dtype, reinterpret_cast<hipStream_t>(stream_ptr),
               format);
@@ -1801,8 +1863,8 @@ ArcW4A16Plan silu_mul_plan(int batch, int n, int k, int group_size, int cu_count
   if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/true, cus, given)) {
     return plan;
   }
-  if (with_workspace && tile_takes_fused(batch, n, k) &&
-      tile_plan(plan, batch, n, k, group_size, /*silu=*/true, cus)) {
+  if (with_workspace && tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
+                                  fused_dot2_us(batch, n, k, group_size, /*silu=*/true, cus))) {
     return plan;
   }
   plan = ArcW4A16Plan{};
@@ -1870,8 +1932,8 @@ ArcW4A16Plan plan_w4a16_fused(int batch, int n, int k, int group_size, int activ
   if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/false, cus, given)) {
     return plan;
   }
-  if (tile_takes_fused(batch, n, k) &&
-      tile_plan(plan, batch, n, k, group_size, /*silu=*/false, cus)) {
+  if (tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
+                fused_dot2_us(batch, n, k, group_size, /*silu=*/false, cus))) {
     return plan;
   }
   return plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, cu_count,
@@ -1894,7 +1956,7 @@ void w4a16_forward_fused(std::uintptr_t activations_ptr, std::uintptr_t norm_wei
       plan_w4a16_fused(batch, n, k, group_size, activation_dtype, 0, packet_format, silu);
   validate_workspace(plan, workspace_ptr, workspace_bytes);
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  if (plan.schedule == kScheduleTiles) {
+  if (is_tile_schedule(plan.schedule)) {
     run_tiles(activations_ptr, packets_ptr, output_ptr, reinterpret_cast<void*>(workspace_ptr),
               batch, n, k, group_size, activation_dtype, stream, format, silu, norm_weight_ptr, eps);
     return;

@@ -56,7 +56,8 @@ CASES = [
     (2, 2048, 32, 128, (16, 2)), (4, 6144, 32, 128, (16, 2)), (5, 1024, 16, 128, (16, 2)),
     (8, 28672, 32, 128, (16, 2)), (9, 14336, 32, 64, (16, 2)), (16, 16384, 32, 128, (16, 2)),
     (3, 8192, 86, 128, (32, 3)), (6, 4096, 21, 128, (32, 3)), (16, 11008, 43, 64, (32, 3)),
-    (17, 512, 8, 128, (32, 3)), (40, 2304, 33, 64, (64, 3)), (130, 1024, 16, 128, None),
+    (17, 512, 33, 128, (32, 3)), (40, 2304, 65, 64, (64, 3)), (130, 1024, 16, 128, None),
+    (40, 512, 8, 128, (8, 0)),
 ]
 
 

@@ -64,22 +64,33 @@ def _check(case, y: torch.Tensor, cols: np.ndarray) -> None:
     assert np.all(err <= bar), f"max error {err.max():.4g}"
 
 
-# rows, columns, groups: edges of the tiles (32, 64, 128 rows; 128 and 256 columns; units of 8 or
-# 16 groups), one group, K split and not, more rows than one launch takes
-SHAPES = [(17, 128, 1), (32, 256, 3), (33, 384, 17), (64, 1152, 21), (65, 640, 40), (129, 256, 33),
-          (200, 4224, 8), (1025, 128, 5)]
+# rows, columns, groups by group size, then (m_tile, K split): edges of the tiles (32, 64, 128 rows; 128
+# and 256 columns; units of 8 or 16 groups) and one group, among shapes the 16-row tiles are slower
+# at; more rows than one launch takes
+SHAPES = {
+    64: [(17, 16512, 9, (32, False)), (32, 2176, 129, (32, True)), (64, 8320, 40, (64, True)),
+         (129, 2176, 129, (64, True)), (300, 6272, 21, (64, False)), (300, 16512, 1, (128, False)),
+         (512, 6272, 21, (128, True)), (1025, 3200, 40, (128, True))],
+    128: [(17, 128, 8, (32, False)), (24, 640, 40, (32, True)), (32, 128, 17, (32, True)),
+          (33, 6272, 33, (64, True)), (64, 16512, 8, (64, False)), (96, 3200, 33, (64, True)),
+          (300, 6272, 3, (64, False)), (200, 16512, 1, (128, False)), (512, 4224, 17, (128, True)),
+          (1025, 640, 65, (64, True))],
+}
 
 
 @pytest.mark.parametrize("fmt", list(FORMATS))
-@pytest.mark.parametrize("group_size", [64, 128])
 @pytest.mark.parametrize("act", ["f16", "bf16"])
-@pytest.mark.parametrize("rows,n,groups", SHAPES)
-def test_row_tiles_match_oracle(rows, n, groups, act, group_size, fmt) -> None:
+@pytest.mark.parametrize("rows,n,groups,group_size,want",
+                         [(*s[:3], g, s[3]) for g, shapes in SHAPES.items() for s in shapes])
+def test_row_tiles_match_oracle(rows, n, groups, group_size, want, act, fmt) -> None:
     case = make_case(rows, n, groups * group_size, group_size, act=act,
                      asymmetric=fmt != "native_sym", seed=rows + n + groups)
     plan = arc_w4a16_plan(batch=rows, n=n, k=case.k, group_size=group_size,
                           activation_dtype=DTYPES[act], packet_format=FORMATS[fmt])
-    assert plan["schedule"] == 3, plan
+    assert plan["schedule"] == (4 if rows <= 32 else 3), plan
+    on_256_cus = arc_w4a16_plan(batch=rows, n=n, k=case.k, group_size=group_size, cu_count=256,
+                                activation_dtype=DTYPES[act], packet_format=FORMATS[fmt])
+    assert (on_256_cus["m_tile"], on_256_cus["max_tile_contributors"] > 1) == want
     x = _tensor(case.x, DTYPES[act])
     packets = _packets(case, fmt)
     y = _forward(case, x, packets, fmt)
@@ -91,11 +102,13 @@ def test_row_tiles_match_oracle(rows, n, groups, act, group_size, fmt) -> None:
     _check(case, y, np.unique(np.linspace(0, n - 1, min(n, 96)).astype(int)))
 
 
-@pytest.mark.parametrize("rows,n,groups", [(40, 512, 40), (20, 256, 64)])
+@pytest.mark.parametrize("rows,n,groups", [(20, 256, 64), (96, 3200, 33)])
 def test_row_tiles_in_a_graph(rows, n, groups) -> None:
     """A captured call (K split, so with counters and partial tiles) replays to the eager bits, with
     eager work in between."""
     case = make_case(rows, n, groups * 128, 128, act="bf16", seed=7)
+    assert arc_w4a16_plan(batch=rows, n=n, k=case.k, group_size=128, activation_dtype=torch.bfloat16,
+                          packet_format=1)["schedule"] == (4 if rows <= 32 else 3)
     x = _tensor(case.x, torch.bfloat16)
     packets = _packets(case, "native_sym")
     want = _forward(case, x, packets, "native_sym")
@@ -113,10 +126,11 @@ def test_row_tiles_in_a_graph(rows, n, groups) -> None:
 
 @pytest.mark.parametrize("fmt", list(FORMATS))
 @pytest.mark.parametrize("exponent", [-100, 100, 120])
-def test_row_tiles_at_the_ends_of_bf16(exponent, fmt) -> None:
+@pytest.mark.parametrize("rows,n,groups", [(18, 256, 64), (96, 3200, 33)])
+def test_row_tiles_at_the_ends_of_bf16(rows, n, groups, exponent, fmt) -> None:
     """Activations scaled by 2^exponent scale the outputs: to 2^120, where sums of (128 + q) x pass
     the largest fp32, and a row with an infinity is not finite while the others are untouched."""
-    case = make_case(18, 256, 512, 128, act="bf16", asymmetric=fmt != "native_sym", seed=5)
+    case = make_case(rows, n, groups * 128, 128, act="bf16", asymmetric=fmt != "native_sym", seed=5)
     x = _tensor(case.x, torch.bfloat16)
     packets = _packets(case, fmt)
     want = _forward(case, x, packets, fmt)
@@ -130,5 +144,5 @@ def test_row_tiles_at_the_ends_of_bf16(exponent, fmt) -> None:
     scaled[3, 17] = math.inf
     again = _forward(case, scaled, packets, fmt)
     assert not torch.isfinite(again[3]).any()
-    keep = [r for r in range(18) if r != 3]
+    keep = [r for r in range(rows) if r != 3]
     assert torch.equal(again[keep], got[keep])
