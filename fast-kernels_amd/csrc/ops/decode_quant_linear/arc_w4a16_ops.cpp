@@ -381,13 +381,23 @@ constexpr long long kMfmaFusedMinSlices = 64;
 bool fused_mfma_takes_small(int batch, bool silu) {
   return batch >= 5 && (batch <= 8 || silu);
 }
-// Fewest weights from which a fused neighbour that the stream kernels do not take (long K, slices
-// that do not divide) goes from the dot2 kernels to the row-tile GEMM, whose two launches take 13 us
-// at least: RMSNorm + 10240 x 8192 at 2 / 4 / 8 rows 19.2 / 29.2 / 68.9 us against 22.7 at any,
-// RMSNorm + 8192 x 11008 G64 + SiLU 34 / 54 / 94 against 26.8, 1024 x 2048 at 8-16 rows 12.0
-// against 13.1, 2048 x 4096 G64 at 8 rows 15.9 against 15.2.
-long long tile_fused_min_weights(int batch) {
-  return batch >= 5 ? 4LL << 20 : batch >= 3 ? 32LL << 20 : 84LL << 20;
+// Whether a fused neighbour at 2-16 rows that the stream kernels do not take (long K, slices that do
+// not divide) goes from the dot2 kernels, which split K, to the row-tile GEMM, whose two launches
+// take 13 us at least. us on MI355X, bf16, dot2 and row tiles: RMSNorm at 2 rows 8192 x 11008 G128
+// 16.9 and 23.5, 53248 x 8192 62.4 and 64.5; at 3 rows 14336 x 5120 G128 20.9 and 21.4, 10240 x 8192
+// G128 28.4 and 22.5, 8192 x 11008 G64 25.3 and 26.0, 12288 x 12288 G64 42.8 and 36.5. With SiLU,
+// where a dot2 workgroup has a pair of slices over all of K: at 2 rows 6144 x 8192 22.9 and 20.1, 10240
+// x 8192 25.1 and 25.4, 28672 x 8192 G64 38.5 and 44.9; at 3 rows 5632 x 7168 33.3 and 19.7. From 5
+// rows: 1024 x 2048 12.0 and 13.1, 2048 x 4096 G64 at 8 rows 15.9 and 15.2.
+bool fused_tiles_take(int batch, int n, int k, int group_size, bool silu, int cu_count) {
+  const long long weights = static_cast<long long>(n) * k;
+  if (batch >= 5) {
+    return weights >= 4LL << 20;
+  }
+  if (silu) {
+    return weights >= 32LL << 20 && (batch >= 3 || n / (2 * fk::kSliceCols) <= cu_count / 2);
+  }
+  return batch >= 3 && weights >= (group_size == 64 ? 96LL : 76LL) << 20;
 }
 // What a fused neighbour takes on the dot2 kernels, in us, for tile_plan. From 17 rows: rounds of
 // workgroups of 8 rows and one slice (SiLU: a pair of slices) over all of K, one (G128) or two (G64)
@@ -397,8 +407,7 @@ long long tile_fused_min_weights(int batch) {
 // and 13.6), two are not (2048 x 1024 18.7 and 14.1).
 double fused_dot2_us(int batch, int n, int k, int group_size, bool silu, int cu_count) {
   if (batch < kTileMinBatch) {
-    const bool tiles =
-        batch >= 2 && static_cast<long long>(n) * k >= tile_fused_min_weights(batch);
+    const bool tiles = batch >= 2 && fused_tiles_take(batch, n, k, group_size, silu, cu_count);
     return tiles ? std::numeric_limits<double>::infinity() : 0.0;
   }
   const double kk = k / 1024.0;
