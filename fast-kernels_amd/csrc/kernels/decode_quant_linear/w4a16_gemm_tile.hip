@@ -1,5 +1,5 @@
-// W4A16 GEMM over row tiles on the gfx950 matrix cores: 17 activation rows and more (batched
-// serving, chunks of a prompt), over reference packets or native slabs.
+// W4A16 GEMM over row tiles on the gfx950 matrix cores: 8-16 activation rows that the stream kernel
+// does not take, 17 and more (batched serving, chunks of a prompt), over reference packets or native slabs.
 //
 // Above 32 rows, and under a fused neighbour, a first launch (tile_prepare_kernel) writes the activations in the order the tiles read them:
 // re-paired (x0,x4)(x1,x5)(x2,x6)(x3,x7) like the code words unpack, [32-row block][group][16-byte

@@ -93,9 +93,9 @@ struct ArcW4A16Plan {
 // slices at once (slice_cols 64); kScheduleStream: one-row native plans on a persistent grid,
 // each workgroup streaming one contiguous range of slabs across slices with the whole activation
 // row staged in LDS (w4a16_gemv_stream.hip).
-// kScheduleTiles: 17 rows and more on the row-tile GEMM (w4a16_gemm_tile.hip): m_tile x slice_cols
-// tiles, K in max_tile_contributors splits; kScheduleTilesDirect: the same with the activations staged
-// by the tiles, without a launch that prepares them.
+// kScheduleTiles: 33 rows and more on the row-tile GEMM (w4a16_gemm_tile.hip): m_tile x slice_cols
+// tiles, K in max_tile_contributors splits; kScheduleTilesDirect: 8 to 32 rows, staged by the
+// tiles, without a launch that prepares them.
 enum Schedule : int {
   kScheduleRuns = 0,
   kSchedulePairs = 1,

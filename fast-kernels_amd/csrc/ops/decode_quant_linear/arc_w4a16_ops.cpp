@@ -153,11 +153,13 @@ constexpr int kMinRowsRunGroups = 16;
 constexpr int kMaxSlicesPerTile = 4;
 // Longest K for which one-row native plans stream slice pairs.
 constexpr int kMaxPairK = 4096;
-// Fewest rows the row-tile GEMM takes from the automatic dispatch: what the 2-16-row kernels, which
-// read the weights once for up to 16 rows, do not take. Among those the 16-row tiles keep the calls
-// they are estimated to be faster at: few columns and little K, where a launch is mostly start-up and
-// the chip has room for a workgroup per 16 rows (16-row and row tiles, 64 rows, bf16, G128: 2048 x
-// 1024 8.1 and 12.9 us, 4864 x 4096 19.6 and 18.5, 16384 x 4096 34.6 and 24.4).
+// The row-tile GEMM takes, from the automatic dispatch, calls of the 16-row tiles (from 8-9 rows, where
+// the stream kernels do not take them, and all from kTileMinBatch rows) that it is estimated to be
+// faster at. The 16-row tiles keep those of few columns and little K, where a launch is mostly
+// start-up and the chip has room for a workgroup per 16 rows (16-row and row tiles, 64 rows, bf16,
+// G128: 2048 x 1024 8.1 and 12.9 us, 4864 x 4096 19.6 and 18.5, 16384 x 4096 34.6 and 24.4). At 8-16
+// rows the row tiles gain from the finer K splits (9 rows: 2432 x 5504 20.7 and 11.3; 12 rows: 4480 x
+// 20224 27.1 and 20.8; 13 rows: 8448 x 16000 28.4 and 28.0).
 constexpr int kTileMinBatch = 17;
 // Most rows whose activations the tiles stage themselves: the 32-row tile's, where the launch that
 // prepares them costs more than every workgroup pairing its own (32 rows, bf16, native_sym, prepared
@@ -256,13 +258,15 @@ ArcW4A16Plan plan_arc_w4a16_for_cu_count(int batch, int n, int k, int group_size
   validate_dimensions(batch, n, k, group_size);
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, fk::gemv_m_tile_for_batch(batch));
-  if (split_k_slices == 0 && batch >= kTileMinBatch &&
+  if (arc_mfma_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true)) {
+    return plan;
+  }
+  if (split_k_slices == 0 && plan.m_tile == fk::kMfmaRows &&
       tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
                 row16_us(plan, group_size, cu_count))) {
     return plan;
   }
-  if (!arc_mfma_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true) &&
-      !arc_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true)) {
+  if (!arc_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true)) {
     arc_quarter_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true);
   }
   return plan;
@@ -887,17 +891,18 @@ double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
   } const c = group_size == 64 ? decltype(c){4.4, 3.76, 1.45, 0.685, 1.9}
                                : decltype(c){4.9, 3.88, 1.87, 0.685, 1.9};
   const int more_rounds = (plan.workgroups + cu_count - 1) / cu_count - 1;
-  return c.first + c.round * more_rounds +
-         c.per_1024_k * plan.groups_per_workgroup * group_size / 1024 *
-             (1 + c.round_k * more_rounds) +
+  const double kk = plan.groups_per_workgroup * group_size / 1024.0;
+  // K of up to 1024 is loaded at once: 1.4 us under the line
+  return c.first - (kk <= 1 ? 1.4 : 0.0) + c.round * more_rounds +
+         c.per_1024_k * kk * (1 + c.round_k * more_rounds) +
          (plan.max_tile_contributors > 1 ? c.fix : 0.0);
 }
 
 // The row-tile GEMM (w4a16_gemm_tile.hip). plain: no fused neighbour; up to kTileDirectMaxRows rows
 // are then staged by the tiles themselves (kScheduleTilesDirect), without the launch that prepares
 // them. More than kTileMaxRows rows run as several launches over one workspace. False (plan
-// unchanged) when the tiles outnumber the fix-up counters, or are not estimated to be faster than
-// another kernel's other_us.
+// unchanged) when the tiles outnumber the fix-up counters, are not estimated to be faster than another
+// kernel's other_us, or need more workspace than a plain plan of up to 16 rows may.
 bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
                int cu_count, double other_us) {
   const bool direct = tile_direct(batch, plain);
@@ -913,7 +918,8 @@ bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool
     us += r.us;
   }
   if (static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters ||
-      us > kTileMargin * other_us) {
+      us > kTileMargin * other_us ||
+      (plain && batch < kTileMinBatch && bytes > kNoAllocScratchBytes)) {
     return false;
   }
   plan = ArcW4A16Plan{};
@@ -939,16 +945,17 @@ ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int a
   }
   ArcW4A16Plan plan = plan_arc_impl(batch, n, k, group_size, activation_dtype, split_k_slices,
                                     cu_count, m_tile_for_kernel(batch, kernel));
-  if (plain && tiles && split_k_slices == 0 && batch >= kTileMinBatch && kernel == kKernelAuto &&
-      tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
-                row16_us(plan, group_size, cu_count))) {
-    return plan;
-  }
   if (plain && split_k_slices == 0 && batch >= kMfmaStreamMinBatch &&
       batch <= kMfmaStreamMaxBatch && kernel != kKernelDot2 && mfma_stream_enabled() &&
       (format != fk::PacketFormat::kArc || arc_mfma_stream_enabled()) &&
       mfma_stream_plan(plan, batch, n, k, group_size, format == fk::PacketFormat::kArc, cu_count,
                        cu_count_given)) {
+    return plan;
+  }
+  if (plain && tiles && split_k_slices == 0 && kernel == kKernelAuto &&
+      plan.m_tile == fk::kMfmaRows &&
+      tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
+                row16_us(plan, group_size, cu_count))) {
     return plan;
   }
   if (format == fk::PacketFormat::kArc && plain && kernel != kKernelMfma &&
@@ -1799,7 +1806,7 @@ void w4a16_forward_noalloc(std::uintptr_t activations_ptr, std::uintptr_t packet
   validate_activation_dtype(activation_dtype);
   validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  // The plan of arc_w4a16_forward_native, checked against the scratch size before any device
+  // The plan of arc_w4a16_forward_native without the row tiles, checked against the scratch size before any device
   // work; then the set-up on the first call on a device (address lookup, counter clear), and the
   // launch with the scratch array standing in for the workspace.
   const ArcW4A16Plan plan =

@@ -127,13 +127,13 @@ typedef struct fk_arc_w4a16_plan {
 #define FK_SCHEDULE_RUNS 0
 #define FK_SCHEDULE_PAIRS 1
 #define FK_SCHEDULE_STREAM 2
-/* FK_SCHEDULE_TILES: 17 rows and more, where it is estimated to be the fastest, and fused neighbours
- * of 2 and more on the row-tile GEMM. m_tile x slice_cols is a workgroup's
+/* FK_SCHEDULE_TILES: 33 rows and more, and fused neighbours of 2 and more, on the row-tile GEMM where
+ * that is estimated to be the fastest. m_tile x slice_cols is a workgroup's
  * tile, max_tile_contributors the K splits; the workspace holds the activations as the tiles read
  * them (of up to 1024 rows at a time) besides the counters and partial tiles, and need not be
  * zero-filled. */
 #define FK_SCHEDULE_TILES 3
-/* FK_SCHEDULE_TILES_DIRECT: the same up to 32 rows with the activations staged by the tiles; the
+/* FK_SCHEDULE_TILES_DIRECT: the same at 8 to 32 rows with the activations staged by the tiles; the
  * workspace is the counters and partial tiles only (none without K splits), zero-filled as
  * fk_arc_w4a16_forward_ex asks. */
 #define FK_SCHEDULE_TILES_DIRECT 4

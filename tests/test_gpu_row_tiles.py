@@ -1,4 +1,4 @@
-"""The row-tile GEMM (17 rows and more) against the CPU oracle: every tile height, K with and without
+"""The row-tile GEMM (8 rows and more) against the CPU oracle: every tile height, K with and without
 splits, ragged rows, columns and groups, each packet format, group size and activation type; captured
 calls; activations near the ends of bf16."""
 
@@ -68,12 +68,12 @@ def _check(case, y: torch.Tensor, cols: np.ndarray) -> None:
 # and 256 columns; units of 8 or 16 groups) and one group, among shapes the 16-row tiles are slower
 # at; more rows than one launch takes
 SHAPES = {
-    64: [(17, 16512, 9, (32, False)), (32, 2176, 129, (32, True)), (64, 8320, 40, (64, True)),
+    64: [(17, 16512, 33, (32, False)), (32, 2176, 129, (32, True)), (64, 8320, 40, (64, True)),
          (129, 2176, 129, (64, True)), (300, 6272, 21, (64, False)), (300, 16512, 1, (128, False)),
          (512, 6272, 21, (128, True)), (1025, 3200, 40, (128, True))],
-    128: [(17, 128, 8, (32, False)), (24, 640, 40, (32, True)), (32, 128, 17, (32, True)),
+    128: [(9, 128, 21, (32, True)), (16, 2432, 33, (32, True)), (17, 16512, 9, (32, False)), (24, 640, 40, (32, True)), (32, 128, 17, (32, True)),
           (33, 6272, 33, (64, True)), (64, 16512, 8, (64, False)), (96, 3200, 33, (64, True)),
-          (300, 6272, 3, (64, False)), (200, 16512, 1, (128, False)), (512, 4224, 17, (128, True)),
+          (300, 6272, 9, (64, False)), (200, 16512, 1, (128, False)), (512, 4224, 17, (128, True)),
           (1025, 640, 65, (64, True))],
 }
 
