@@ -1,4 +1,5 @@
-// W4A16 small-batch GEMM (8-16 activation rows) on the gfx950 matrix cores.
+// W4A16 small-batch GEMM (16-row tiles) on the gfx950 matrix cores: 8-16 rows, and more where the
+// weights are few.
 //
 // Same math and packet formats as w4a16_gemv.hip; with 8 or more rows the dot2 loop there is bound
 // by VALU issue (four v_dot2 per code word per row), so here the products run on

@@ -193,7 +193,7 @@ void arc_w4a16_forward_native(std::uintptr_t activations_ptr, std::uintptr_t pac
                               int packet_format, int activation_dtype, int split_k_slices,
                               std::uintptr_t stream_ptr);
 
-// Kernel choice: the automatic dispatch (dot2 loop below 8 rows, matrix cores from 8), the dot2
+// Kernel choice: the automatic dispatch (dot2 loop, matrix cores, row tiles), the dot2
 // loop for every batch (m-tiles of at most 8 rows), or the matrix-core kernel for every batch
 // (16-row m-tiles over whole 128-column tiles). The suites time each against the others.
 enum KernelChoice : int { kKernelAuto = 0, kKernelDot2 = 1, kKernelMfma = 2 };

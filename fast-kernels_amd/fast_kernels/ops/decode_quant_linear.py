@@ -47,7 +47,7 @@ _ARC_IMPL_WGMMA = "wgmma"
 _ARC_IMPL_MFMA = "mfma"
 _ARC_IMPLS = {_ARC_IMPL_AUTO, _ARC_IMPL_SCALAR, _ARC_IMPL_TC, _ARC_IMPL_WGMMA, _ARC_IMPL_MFMA}
 # Kernel choice of the HIP GEMV per impl (FK_KERNEL_* in include/fk_w4a16.h): "auto" dispatches
-# by batch (dot2 loop below 8 rows, matrix cores from 8), "scalar" is the dot2 (FMA) loop for every
+# by batch (dot2 loop, matrix cores, row tiles), "scalar" is the dot2 (FMA) loop for every
 # batch, "mfma" the matrix-core kernel for every batch.
 KERNEL_AUTO, KERNEL_DOT2, KERNEL_MFMA = 0, 1, 2
 _IMPL_KERNEL = {_ARC_IMPL_AUTO: KERNEL_AUTO, _ARC_IMPL_SCALAR: KERNEL_DOT2,
