@@ -1,13 +1,14 @@
 // W4A16 GEMM over row tiles on the gfx950 matrix cores: 8-16 activation rows that the stream kernel
 // does not take, 17 and more (batched serving, chunks of a prompt), over reference packets or native slabs.
 //
-// Above 32 rows, and under a fused neighbour, a first launch (tile_prepare_kernel) writes the activations in the order the tiles read them:
-// re-paired (x0,x4)(x1,x5)(x2,x6)(x3,x7) like the code words unpack, [32-row block][group][16-byte
-// unit][row], so staging is a straight copy and every LDS access is 512 consecutive bytes per
-// half wave; beside them the (row, group) sums. It applies the RMSNorm where one is fused, so
-// that costs no pass of its own. Up to 32 plain rows the tiles stage the activations themselves: the
-// launch costs 4-5 us there and the pairing little (32 rows, bf16 native: 28672 x 4096 23.6 -> 22.1
-// us, 4096 x 14336 18.9 -> 16.0, 10240 x 8192 21.1 -> 18.1, 4096 x 4096 12.9 -> 11.0).
+// Above 32 rows, and under a fused neighbour, a first launch (tile_prepare_kernel) writes the
+// activations in the order the tiles read them: re-paired (x0,x4)(x1,x5)(x2,x6)(x3,x7) like the code
+// words unpack, [32-row block][group][16-byte unit][row], so staging is a straight copy and every
+// LDS access is 512 consecutive bytes per half wave; beside them the (row, group) sums. It applies
+// the RMSNorm where one is fused, so that costs no pass of its own. Up to 32 plain rows the tiles
+// stage the activations themselves: the launch costs 4-5 us there and the pairing little (32 rows,
+// bf16 native: 28672 x 4096 23.6 -> 22.1 us, 4096 x 14336 18.9 -> 16.0, 10240 x 8192 21.1 -> 18.1,
+// 4096 x 4096 12.9 -> 11.0).
 //
 // The GEMM's workgroup (8 waves) owns BM rows x BN columns. Each wave owns whole 32-column slices
 // of the tile, reads their code words straight into registers (each word is unpacked once per

@@ -1806,9 +1806,9 @@ void w4a16_forward_noalloc(std::uintptr_t activations_ptr, std::uintptr_t packet
   validate_activation_dtype(activation_dtype);
   validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  // The plan of arc_w4a16_forward_native without the row tiles, checked against the scratch size before any device
-  // work; then the set-up on the first call on a device (address lookup, counter clear), and the
-  // launch with the scratch array standing in for the workspace.
+  // The plan of arc_w4a16_forward_native without the row tiles, checked against the scratch size
+  // before any device work; then the set-up on the first call on a device (address lookup, counter
+  // clear), and the launch with the scratch array standing in for the workspace.
   const ArcW4A16Plan plan =
       plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, device_cu_count(),
                            packet_format, kKernelAuto, /*plain=*/true, /*tiles=*/false);
