@@ -1472,7 +1472,8 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
   ArcW4A16Plan plan =
       plan_arc_w4a16_for_cu_count(batch, n, k, group_size, kActivationF16, 0, device_cu_count());
-  if (is_tile_schedule(plan.schedule) && !library_workspace_ready(plan.workspace_bytes, stream)) {
+  if (is_tile_schedule(plan.schedule) && plan.workspace_bytes > 0 &&
+      !library_workspace_ready(plan.workspace_bytes, stream)) {
     // A captured call cannot allocate: the per-tile kernels need no prepared activations (and no
     // workspace at all for most shapes).
     plan = plan_for_format_impl(batch, n, k, group_size, kActivationF16, 0, device_cu_count(),
