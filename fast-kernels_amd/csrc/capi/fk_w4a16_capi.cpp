@@ -70,6 +70,10 @@ int fk_arc_w4a16_forward(const void* activations, const void* packets, const voi
   });
 }
 
+int fk_w4a16_release_workspaces(void) {
+  return guarded([] { ops::release_workspaces(); });
+}
+
 int fk_arc_w4a16_forward_split_k(const void* activations, const void* packets,
                                  const void* group_sums, void* partials, int batch, int n, int k,
                                  int group_size, int packet_stride_bytes, int split_k_slices,

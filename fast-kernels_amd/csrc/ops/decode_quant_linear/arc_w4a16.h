@@ -27,6 +27,10 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
                        std::uintptr_t group_sums_ptr, std::uintptr_t output_ptr, int batch, int n,
                        int k, int group_size, int packet_stride_bytes, std::uintptr_t stream_ptr);
 
+// Frees what arc_w4a16_forward keeps for calls of many rows (prepared activations and partial tiles:
+// up to 96 MB for each of the last eight streams); the next such call allocates again.
+void release_workspaces();
+
 void arc_w4a16_forward_split_k(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
                                std::uintptr_t group_sums_ptr, std::uintptr_t partials_ptr,
                                int batch, int n, int k, int group_size, int packet_stride_bytes,

@@ -72,6 +72,13 @@ void validate_dimensions(int batch, int n, int k, int group_size) {
   }
 }
 
+// The kernels index stream-K units (row tile, 32-column slice, group) in 32 bits.
+void validate_units(int batch, int n, int k, int group_size) {
+  if (static_cast<long long>(n / 32) * batch * (k / group_size) >= (1LL << 31)) {
+    throw_invalid("W4A16: batch * (n / 32) * (k / group_size) must stay below 2^31");
+  }
+}
+
 void validate_packet_stride(int group_size, int packet_stride_bytes) {
   const int expected = fk::packet_stride_bytes(group_size);
   if (packet_stride_bytes != expected) {
@@ -933,6 +940,25 @@ bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool
   return true;
 }
 
+// Rows per launch of a plain row-tile call whose launches' workspace is at most `limit` bytes, and
+// that workspace; 0 where not even 128 rows fit.
+int tile_rows_within(int batch, int n, int k, int group_size, int cu_count, std::size_t limit,
+                     std::size_t& bytes) {
+  for (int rows = std::min(batch, fk::kTileMaxRows);; rows = std::max(rows / 2, 128)) {
+    const bool direct = tile_direct(batch, /*plain=*/true);
+    const auto need = [&](int r) {
+      return fk::tile_shape(r, n, k, group_size, direct, cu_count, kCounterRegionBytes).end;
+    };
+    bytes = std::max(need(rows), batch % rows != 0 ? need(batch % rows) : 0);
+    if (bytes <= limit) {
+      return rows;
+    }
+    if (rows <= 128) {
+      return 0;
+    }
+  }
+}
+
 // plan_w4a16_for_format for a kernel choice (kKernelDot2 is what the fused kernels need).
 ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int activation_dtype,
                                   int split_k_slices, int cu_count, int packet_format,
@@ -1137,65 +1163,122 @@ ArcW4A16Plan plan_w4a16_for_kernel(int batch, int n, int k, int group_size, int 
 
 namespace {
 
-// Library-owned fix-up workspace for the reference-signature forward, which has no workspace
-// argument: one per (device, stream), so that calls on different streams never share counters or
-// partials. Grown on demand (so the first call for a larger shape on a stream allocates and must
-// not run under stream capture): the old buffer is freed after synchronising its stream, its only
-// user. The counter region is zeroed, stream-ordered, at allocation, and the kernel leaves it
-// zeroed. (The reference shares one cached group_sums buffer across streams instead,
-// decode_quant_linear.py:150-168.)
-struct StreamWorkspace {
+// Allocations by this thread while another stream, or another thread, captures a graph in the
+// global capture mode, which would otherwise refuse them and break that capture.
+class RelaxedCaptureScope {
+ public:
+  RelaxedCaptureScope() { check_hip(hipThreadExchangeStreamCaptureMode(&mode_), "capture mode"); }
+  ~RelaxedCaptureScope() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  RelaxedCaptureScope(const RelaxedCaptureScope&) = delete;
+  RelaxedCaptureScope& operator=(const RelaxedCaptureScope&) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
+bool stream_is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  check_hip(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
+  return status != hipStreamCaptureStatusNone;
+}
+
+// Memory of the reference-signature forward, which has no workspace argument. (The reference shares
+// one cached group_sums buffer across streams instead, decode_quant_linear.py:150-168.) Two kinds:
+//
+//  * Fix-up workspaces (K splits of the 1- to 16-row kernels; a few MB): one per (device, stream), so
+//    that calls on different streams never share counters or partials. Grown on demand, so the first
+//    call for a larger shape on a stream allocates and cannot be captured. A buffer that a captured
+//    call has taken is never freed: the graph replays into it (replays, like the calls, belong on that
+//    stream). The counter region is zeroed, stream-ordered, at allocation, and the kernels leave it
+//    zeroed.
+//  * Row-tile workspaces (prepared activations, partial tiles; up to kTileWorkspaceBytes): the last
+//    kTileWorkspaces (device, stream)s that took one. Captured calls never take one (arc_w4a16_forward),
+//    so the longest unused is freed when another stream needs one, and release_workspaces frees all.
+//
+// Both are handed out locked: the lock is held until the launches that use the memory are enqueued,
+// so that no other thread frees it between.
+struct FixupWorkspace {
+  void* ptr = nullptr;
+  std::size_t bytes = 0;
+  bool captured = false;
+};
+struct TileWorkspace {
+  int device = 0;
+  hipStream_t stream = nullptr;
   void* ptr = nullptr;
   std::size_t bytes = 0;
 };
+constexpr std::size_t kTileWorkspaces = 8;
+constexpr std::size_t kTileWorkspaceBytes = 96u << 20;
 
-struct StreamWorkspaces {
-  std::map<std::pair<int, hipStream_t>, StreamWorkspace> spaces;
+struct LibraryMemory {
   std::mutex mutex;
+  std::map<std::pair<int, hipStream_t>, FixupWorkspace> fixups;
+  std::vector<TileWorkspace> tiles;  // the last used at the back
 };
 
-StreamWorkspaces& stream_workspaces() {
-  static StreamWorkspaces all;
-  return all;
+LibraryMemory& library_memory() {
+  static LibraryMemory* const all = new LibraryMemory;  // outlives every thread's last call
+  return *all;
 }
 
-// Whether library_workspace(bytes, stream) can be had now: it is large enough already, or the
-// stream is not being captured.
-bool library_workspace_ready(std::size_t bytes, hipStream_t stream) {
+int current_device() {
   int device = 0;
   check_hip(hipGetDevice(&device), "hipGetDevice");
-  {
-    StreamWorkspaces& all = stream_workspaces();
-    std::lock_guard<std::mutex> lock(all.mutex);
-    const auto it = all.spaces.find({device, stream});
-    if (it != all.spaces.end() && it->second.bytes >= bytes) {
-      return true;
-    }
-  }
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  check_hip(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
-  return status == hipStreamCaptureStatusNone;
+  return device;
 }
 
-void* library_workspace(std::size_t bytes, hipStream_t stream) {
-  int device = 0;
-  check_hip(hipGetDevice(&device), "hipGetDevice");
-  StreamWorkspaces& all = stream_workspaces();
-  std::lock_guard<std::mutex> lock(all.mutex);
-  StreamWorkspace& ws = all.spaces[{device, stream}];
+// (library_memory().mutex held)
+void* fixup_workspace(std::size_t bytes, hipStream_t stream, bool capturing) {
+  FixupWorkspace& ws = library_memory().fixups[{current_device(), stream}];
   if (ws.bytes < bytes) {
-    if (ws.ptr != nullptr) {
+    if (capturing) {
+      throw std::runtime_error(
+          "a captured call cannot allocate its workspace: run it once on this stream first");
+    }
+    const RelaxedCaptureScope relaxed;
+    if (ws.ptr != nullptr && !ws.captured) {
       check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
       check_hip(hipFree(ws.ptr), "hipFree");
-      ws.ptr = nullptr;
-      ws.bytes = 0;
     }
+    ws = FixupWorkspace{};
     const std::size_t grown = std::max<std::size_t>(bytes, 1u << 20);
     check_hip(hipMalloc(&ws.ptr, grown), "hipMalloc(workspace)");
     check_hip(hipMemsetAsync(ws.ptr, 0, grown, stream), "hipMemsetAsync(workspace)");
     ws.bytes = grown;
   }
+  ws.captured = ws.captured || capturing;
   return ws.ptr;
+}
+
+// Null where the memory cannot be had. hipFree waits for the device, so for every launch that uses
+// what it frees. (library_memory().mutex held)
+void* tile_workspace(std::size_t bytes, hipStream_t stream) {
+  std::vector<TileWorkspace>& tiles = library_memory().tiles;
+  const int device = current_device();
+  auto it = std::find_if(tiles.begin(), tiles.end(), [&](const TileWorkspace& t) {
+    return t.device == device && t.stream == stream;
+  });
+  if (it != tiles.end() && it->bytes >= bytes) {
+    std::rotate(it, it + 1, tiles.end());
+    return tiles.back().ptr;
+  }
+  const RelaxedCaptureScope relaxed;
+  if (it == tiles.end() && tiles.size() >= kTileWorkspaces) {
+    it = tiles.begin();
+  }
+  if (it != tiles.end()) {
+    void* const old = it->ptr;
+    tiles.erase(it);
+    check_hip(hipFree(old), "hipFree");
+  }
+  TileWorkspace t{device, stream, nullptr, bytes};
+  if (hipMalloc(&t.ptr, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  tiles.push_back(t);
+  return t.ptr;
 }
 
 void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::uintptr_t output_ptr,
@@ -1204,11 +1287,7 @@ void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::u
               fk::PacketFormat format = fk::PacketFormat::kArc,
               fk::GemvFuse fuse = fk::GemvFuse::kNone, std::uintptr_t norm_weight_ptr = 0,
               float eps = 0.0f) {
-  // The kernels index stream-K units (row tile, 32-column slice, group) in 32 bits.
-  const long long units_bound = static_cast<long long>(n / 32) * batch * (k / group_size);
-  if (units_bound >= (1LL << 31)) {
-    throw_invalid("W4A16: batch * (n / 32) * (k / group_size) must stay below 2^31");
-  }
+  validate_units(batch, n, k, group_size);
   fk::GemvLaunch l;
   l.x = reinterpret_cast<const void*>(activations_ptr);
   l.packets = reinterpret_cast<const void*>(packets_ptr);
@@ -1295,16 +1374,17 @@ void run_gemv(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr, std::u
   check_hip(fk::launch_w4a16_gemv(l, stream), "w4a16_gemv launch");
 }
 
-// The launches of a row-tile plan.
+// The launches of a row-tile plan, max_rows rows each.
 void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
                std::uintptr_t output_ptr, void* workspace, int batch, int n, int k, int group_size,
                int activation_dtype, hipStream_t stream, fk::PacketFormat format, bool silu = false,
-               std::uintptr_t norm_weight_ptr = 0, float eps = 0.0f) {
+               std::uintptr_t norm_weight_ptr = 0, float eps = 0.0f,
+               int max_rows = fk::kTileMaxRows) {
   const int cu_count = device_cu_count();
   const bool direct = tile_direct(batch, !silu && norm_weight_ptr == 0);
-  for (int row = 0; row < batch; row += fk::kTileMaxRows) {
+  for (int row = 0; row < batch; row += max_rows) {
     fk::TileLaunch l;
-    l.M = std::min(batch - row, fk::kTileMaxRows);
+    l.M = std::min(batch - row, max_rows);
     l.N = n;
     l.K = k;
     l.group_size = group_size;
@@ -1320,6 +1400,9 @@ void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
     l.eps = eps;
     const fk::TileShape s =
         fk::tile_shape(l.M, n, k, group_size, direct, cu_count, kCounterRegionBytes);
+    if (s.splits > 1 && static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters) {
+      throw std::logic_error("more row tiles with K split than fix-up counters");
+    }
     check_hip(fk::launch_w4a16_gemm_tile(l, s, stream), "w4a16_gemm_tile launch");
   }
 }
@@ -1470,23 +1553,66 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
   validate_packet_stride(group_size, packet_stride_bytes);
   validate_forward_buffers(activations_ptr, packets_ptr, output_ptr);
   const auto stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  const int cus = device_cu_count();
   ArcW4A16Plan plan =
-      plan_arc_w4a16_for_cu_count(batch, n, k, group_size, kActivationF16, 0, device_cu_count());
-  if (is_tile_schedule(plan.schedule) && plan.workspace_bytes > 0 &&
-      !library_workspace_ready(plan.workspace_bytes, stream)) {
-    // A captured call cannot allocate: the per-tile kernels need no prepared activations (and no
-    // workspace at all for most shapes).
-    plan = plan_for_format_impl(batch, n, k, group_size, kActivationF16, 0, device_cu_count(),
-                                kPacketArc, kKernelAuto, /*plain=*/true, /*tiles=*/false);
-  }
-  void* workspace = plan.workspace_bytes > 0 ? library_workspace(plan.workspace_bytes, stream) : nullptr;
+      plan_arc_w4a16_for_cu_count(batch, n, k, group_size, kActivationF16, 0, cus);
+  LibraryMemory& memory = library_memory();
+  std::unique_lock<std::mutex> lock(memory.mutex, std::defer_lock);
   if (is_tile_schedule(plan.schedule)) {
-    run_tiles(activations_ptr, packets_ptr, output_ptr, workspace, batch, n, k, group_size,
-              kActivationF16, stream, fk::PacketFormat::kArc);
-    return;
+    if (plan.workspace_bytes == 0) {
+      run_tiles(activations_ptr, packets_ptr, output_ptr, nullptr, batch, n, k, group_size,
+                kActivationF16, stream, fk::PacketFormat::kArc);
+      return;
+    }
+    // The 16-row tiles need little memory or none, and none that another call may free: they run
+    // where the call is captured or the row tiles' memory cannot be had. An eager call still allocates
+    // what they need, so that it may be captured on this stream afterwards.
+    const ArcW4A16Plan tiles = plan;
+    plan = plan_for_format_impl(batch, n, k, group_size, kActivationF16, 0, cus, kPacketArc,
+                                kKernelAuto, /*plain=*/true, /*tiles=*/false);
+    const bool capturing = stream_is_capturing(stream);
+    lock.lock();
+    if (!capturing) {
+      if (plan.workspace_bytes > 0) {
+        fixup_workspace(plan.workspace_bytes, stream, false);
+      }
+      void* workspace = nullptr;
+      int rows = batch;
+      if (tiles.schedule == kScheduleTilesDirect) {
+        workspace = fixup_workspace(tiles.workspace_bytes, stream, false);  // zeroed counters
+      } else {
+        std::size_t bytes = 0;
+        rows = tile_rows_within(batch, n, k, group_size, cus, kTileWorkspaceBytes, bytes);
+        workspace = rows > 0 ? tile_workspace(bytes, stream) : nullptr;
+      }
+      if (workspace != nullptr) {
+        run_tiles(activations_ptr, packets_ptr, output_ptr, workspace, batch, n, k, group_size,
+                  kActivationF16, stream, fk::PacketFormat::kArc, /*silu=*/false,
+                  /*norm_weight_ptr=*/0, /*eps=*/0.0f, rows);
+        return;
+      }
+    }
+  }
+  void* workspace = nullptr;
+  if (plan.workspace_bytes > 0) {
+    if (!lock.owns_lock()) {
+      lock.lock();
+    }
+    workspace = fixup_workspace(plan.workspace_bytes, stream, stream_is_capturing(stream));
   }
   run_gemv(activations_ptr, packets_ptr, output_ptr, workspace, plan, batch, n, k, group_size,
            kActivationF16, stream);
+}
+
+void release_workspaces() {
+  LibraryMemory& memory = library_memory();
+  const std::lock_guard<std::mutex> lock(memory.mutex);
+  const RelaxedCaptureScope relaxed;
+  while (!memory.tiles.empty()) {
+    void* const ptr = memory.tiles.back().ptr;
+    memory.tiles.pop_back();
+    check_hip(hipFree(ptr), "hipFree");
+  }
 }
 
 void arc_w4a16_forward_split_k(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,

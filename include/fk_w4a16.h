@@ -60,10 +60,16 @@ int fk_compute_arc_w4a16_group_sums(const void* activations, void* sums, int bat
  * group_sums is accepted for signature compatibility and not read (may be NULL): the kernel forms
  * the activation sums it needs itself, in the same launch. Uses a library-owned split-K workspace
  * per (device, stream): calls on different streams never share one, and the first call of a
- * larger shape on a stream allocates (so it must not be the first call under graph capture). */
+ * larger shape on a stream allocates (so it must not be the first call under graph capture). A
+ * captured call keeps that workspace for good, and its graph is to be replayed on that stream.
+ * Eager calls of more rows also hold prepared activations and partial tiles, up to 96 MB for each
+ * of the last eight streams (fk_w4a16_release_workspaces); captured calls run kernels without. */
 int fk_arc_w4a16_forward(const void* activations, const void* packets, const void* group_sums,
                          void* output, int batch, int n, int k, int group_size,
                          int packet_stride_bytes, void* stream);
+
+/* Frees what fk_arc_w4a16_forward holds for eager calls of many rows; the next one allocates again. */
+int fk_w4a16_release_workspaces(void);
 
 /* Reference: arc_w4a16_forward_split_k, arc_w4a16.h:19-22 / arc_w4a16.cu:709-737.
  * Writes fp32 partials[S, batch, n]; slice z covers groups [z*ceil(NG/S), (z+1)*ceil(NG/S)).

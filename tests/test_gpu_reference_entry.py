@@ -53,3 +53,82 @@ def test_captured_call_of_a_plan_without_workspace() -> None:
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+# rows, n, k: row tiles that need prepared activations (no K split and K splits), and ones that need
+# only partial tiles; the 16-row tiles need no memory at the first and the fourth
+CAPTURED = [(33, 22016, 4096), (96, 3200, 4224), (20, 4096, 14336), (300, 2048, 8192)]
+
+
+@pytest.mark.parametrize("rows,n,k", CAPTURED)
+def test_captured_call_survives_larger_calls(rows, n, k) -> None:
+    """A graph of the call replays to the same bits after the stream's memory has grown for calls of
+    more rows, and after that memory is given back; the call captured is the one without row tiles."""
+    x, packets = _case(rows, n, k)
+    more, more_packets = _case(600, 10240, 8192)
+    stream = torch.cuda.Stream()
+    out, more_out = _new_out(x, n), _new_out(more, 10240)
+    torch.cuda.synchronize()
+    _call(x, packets, out, stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        _call(x, packets, out, stream)
+    want = arc_w4a16_forward(x, packets, n=n, k=k, group_size=G, impl="mfma")  # 16-row tiles
+    torch.cuda.synchronize()
+    more_want = None
+    for step in range(4):
+        _call(more, more_packets, more_out, stream)
+        torch.cuda.synchronize()
+        more_want = more_out.clone() if more_want is None else more_want
+        assert torch.equal(more_out, more_want)
+        out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        if step == 1:
+            native_module().release_workspaces()
+
+
+def test_row_tiles_on_many_streams_at_once() -> None:
+    """More streams than the library keeps memory for, calls of two sizes (a K split whose counters
+    and partial tiles must not be shared; more rows than one launch's memory allows) interleaved."""
+    runs = []
+    for rows, n, k in ((96, 3200, 4224), (20, 4096, 14336), (1100, 1024, 57344)):
+        x, packets = _case(rows, n, k)
+        runs.append((x, packets, arc_w4a16_forward(x, packets, n=n, k=k, group_size=G)))
+    streams = [torch.cuda.Stream() for _ in range(10)]
+    torch.cuda.synchronize()
+    for _ in range(2):
+        outs = []
+        for stream in streams:
+            for x, packets, want in runs:
+                out = torch.zeros_like(want)
+                stream.wait_stream(torch.cuda.current_stream())
+                _call(x, packets, out, stream)
+                outs.append((out, want))
+        torch.cuda.synchronize()
+        for out, want in outs:
+            # both round sums of the same products to fp16 once, in another order
+            assert (out.float() - want.float()).abs().max() <= 2.0**-9 * want.float().abs().max()
+    native_module().release_workspaces()
+
+
+def test_eager_call_while_another_stream_captures() -> None:
+    """The first call on a stream allocates; a capture under way on another stream goes on."""
+    x, packets = _case(96, 3200, 4224)
+    want = arc_w4a16_forward(x, packets, n=3200, k=4224, group_size=G)
+    stream = torch.cuda.Stream()
+    out, a = torch.zeros_like(want), torch.ones(1024, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        b = a + 1
+        _call(x, packets, out, stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(b, a + 1)
