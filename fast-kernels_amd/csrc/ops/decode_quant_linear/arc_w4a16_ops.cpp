@@ -1380,6 +1380,7 @@ void run_tiles(std::uintptr_t activations_ptr, std::uintptr_t packets_ptr,
                int activation_dtype, hipStream_t stream, fk::PacketFormat format, bool silu = false,
                std::uintptr_t norm_weight_ptr = 0, float eps = 0.0f,
                int max_rows = fk::kTileMaxRows) {
+  validate_units(batch, n, k, group_size);
   const int cu_count = device_cu_count();
   const bool direct = tile_direct(batch, !silu && norm_weight_ptr == 0);
   for (int row = 0; row < batch; row += max_rows) {

@@ -132,3 +132,18 @@ def test_eager_call_while_another_stream_captures() -> None:
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(b, a + 1)
+
+
+def test_too_many_units_are_refused() -> None:
+    """batch * (n / 32) * (k / group_size) from 2^31 on is refused before any launch, by the row tiles
+    as by the other kernels."""
+    x, packets = _case(17, 57344, 8192)
+    out = _new_out(x, 57344)
+    rows = 2**31 // (57344 // 32 * (8192 // G)) + 1
+    with pytest.raises(ValueError, match="2\\^31"):
+        native_module().arc_w4a16_forward(x.data_ptr(), packets.data_ptr(), 0, out.data_ptr(), rows,
+                                          57344, 8192, G, arc_packet_stride_bytes(G), 0)
+    with pytest.raises(ValueError, match="2\\^31"):
+        native_module().w4a16_forward_fused(x.data_ptr(), x.data_ptr(), 1e-5, packets.data_ptr(),
+                                            out.data_ptr(), packets.data_ptr(), 2**40, rows, 57344,
+                                            8192, G, 1, 0, True, 0)
