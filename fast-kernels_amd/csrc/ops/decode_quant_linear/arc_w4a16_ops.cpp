@@ -175,8 +175,7 @@ constexpr int kTileMinBatch = 17;
 // 34.6).
 constexpr int kTileDirectMaxRows = 32;
 // The row tiles' estimate has to be this part of the other kernel's: the estimates' errors are about
-// 7 % each. Over the 560 shapes they were fitted to, the choice costs 0.3 % against the faster of
-// the two at every shape.
+// 7 % each.
 constexpr double kTileMargin = 0.92;
 bool tile_direct(int batch, bool plain) { return plain && batch <= kTileDirectMaxRows; }
 
@@ -891,18 +890,29 @@ bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group
 }
 
 // Estimated time, in us, of a plan of 16-row tiles: rounds of workgroups, each start-up and groups,
-// and the fix-up of K splits. Fitted like the row tiles' (deviation 6-8 %).
+// and the fix-up of K splits. The lower of two fits. The first, like the row tiles', is to 560 bf16
+// launches over native slabs, in whole rounds (deviation 6-8 %). The second is to 1480 drawn launches of
+// both activation types over all packet formats (9-10 %); runs of up to 3072 values share a CU, so
+// workgroups just past a whole round cost less than another one (39 rows, 11520 x 1920 G128 fp16, 270
+// workgroups: 19.0 us by the first fit, 14.9 measured, the row tiles 17.9). By the first fit alone 13 of
+// the 625 drawn launches on the row tiles were slower there by 3-20 %, by both 8 by up to 11 %.
 double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
-  struct {
-    double first, per_1024_k, round, round_k, fix;
-  } const c = group_size == 64 ? decltype(c){4.4, 3.76, 1.45, 0.685, 1.9}
-                               : decltype(c){4.9, 3.88, 1.87, 0.685, 1.9};
-  const int more_rounds = (plan.workgroups + cu_count - 1) / cu_count - 1;
+  struct Fit {
+    double first, per_1024_k, round, round_per_1024_k, fix, short_k;  // short_k: K up to 1024, loaded at once
+  };
+  const Fit whole = group_size == 64 ? Fit{4.4, 3.76, 1.45, 2.58, 1.9, 1.4}
+                                     : Fit{4.9, 3.88, 1.87, 2.66, 1.9, 1.4};
+  const Fit shared = group_size == 64 ? Fit{6.5, 2.98, 1.59, 3.07, 3.9, 3.5}
+                                      : Fit{6.6, 3.41, 2.34, 2.68, 3.85, 2.5};
+  const double more = (plan.workgroups + cu_count - 1) / cu_count - 1;
+  const double over = std::max(0.0, static_cast<double>(plan.workgroups) / cu_count - 1);
   const double kk = plan.groups_per_workgroup * group_size / 1024.0;
-  // K of up to 1024 is loaded at once: 1.4 us under the line
-  return c.first - (kk <= 1 ? 1.4 : 0.0) + c.round * more_rounds +
-         c.per_1024_k * kk * (1 + c.round_k * more_rounds) +
-         (plan.max_tile_contributors > 1 ? c.fix : 0.0);
+  const auto us = [&](const Fit& c, double rounds) {
+    return c.first - (kk <= 1 ? c.short_k : 0.0) + c.per_1024_k * kk +
+           rounds * (c.round + c.round_per_1024_k * kk) +
+           (plan.max_tile_contributors > 1 ? c.fix : 0.0);
+  };
+  return std::min(us(whole, more), us(shared, kk <= 3 ? (more + over) / 2 : more));
 }
 
 // The row-tile GEMM (w4a16_gemm_tile.hip). plain: no fused neighbour; up to kTileDirectMaxRows rows
