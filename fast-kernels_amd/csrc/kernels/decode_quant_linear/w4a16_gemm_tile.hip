@@ -218,11 +218,6 @@ struct Tile {
   static constexpr int kSUnits = kChunkGroups * kBlocks * kBlockRows;
   static constexpr int kBufUnits = kXUnits + kSUnits;
   static constexpr int kXPer = kXUnits / kTileThreads;
-  // A 32-row tile is the launch's only row tile: no other workgroup reads its weights, and they are
-  // loaded non-temporally. Larger tiles share theirs through the caches (64-row tile, 500 drawn shapes:
-  // 4 % faster than with non-temporal loads at one row tile, 5, 6, 8 and 10 % at 2, 3-4, 5-8 and 9-12;
-  // 370 rows, 4864 x 3328 G128: 31.5 -> 27.1 us).
-  static constexpr bool kOnce = kBlocks == 1;
   static constexpr int kOutPitch = kBN + 8;       // 16-bit elements per staged output row
   static constexpr size_t kLdsBytes = 2 * static_cast<size_t>(kBufUnits) * 16 + 16;
   static constexpr int kAcc = RS * CS * 16;       // accumulators per lane
@@ -238,24 +233,6 @@ struct SliceRegs {
   uint32_t w[G / 16];
   uint32_t alpha;
   uint32_t beta;  // kArc: beta, kNativeAsym: -zp, as fp16 bits
-};
-
-template <bool kOnce>
-struct WeightLoad {
-  static __device__ __forceinline__ uint32_t u16(const uint8_t* p) {
-    return *reinterpret_cast<const uint16_t*>(p);
-  }
-  static __device__ __forceinline__ uint32_t b4(const uint8_t* p) {
-    return kOnce ? stream_load4(p) : *reinterpret_cast<const uint32_t*>(p);
-  }
-  static __device__ __forceinline__ u32x2_t b8(const uint8_t* p) {
-    const u32x2_t* q = reinterpret_cast<const u32x2_t*>(p);
-    return kOnce ? __builtin_nontemporal_load(q) : *q;
-  }
-  static __device__ __forceinline__ u32x4_t b16(const uint8_t* p) {
-    const u32x4_t* q = reinterpret_cast<const u32x4_t*>(p);
-    return kOnce ? __builtin_nontemporal_load(q) : *q;
-  }
 };
 
 // Byte offsets of a lane in a group's slab (native) or packet (kArc, of 32-column quarter 0):
@@ -279,20 +256,24 @@ __device__ __forceinline__ uint32_t lane_scale(int lane) {
              : native_record_offset(G) + native_record_bytes(F) * (c % 16) + 2 * (c / 16);
 }
 
-template <int G, PacketFormat F, bool kOnce>
+// Plain loads: row tiles share the weights through the caches, and a 128-byte line that two slabs
+// share is kept for the second. (Non-temporal ones were 3-5 % slower in the 32-row tile, 5-8 % at G64
+// over native slabs, and 4 % in the 64-row tile with one row tile to 10 % with 9-12; 370 rows, 4864 x
+// 3328 G128: 31.5 -> 27.1 us.)
+template <int G, PacketFormat F>
 __device__ __forceinline__ void load_slice(SliceRegs<G>& r, const uint8_t* group, uint32_t words,
                                            uint32_t scale) {
-  using L = WeightLoad<kOnce>;
+  const auto u16 = [](const uint8_t* p) -> uint32_t { return *reinterpret_cast<const uint16_t*>(p); };
   if constexpr (F == PacketFormat::kArc) {
 #pragma unroll
     for (int v = 0; v < G / 16; ++v) {
-      r.w[v] = L::b4(group + words + v * 2 * kTileCols * 4);
+      r.w[v] = *reinterpret_cast<const uint32_t*>(group + words + v * 2 * kTileCols * 4);
     }
-    r.beta = L::u16(group + scale + kTileCols * 2);
+    r.beta = u16(group + scale + kTileCols * 2);
   } else if constexpr (G == 128) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x4_t v = L::b16(group + words + s * 512);
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(group + words + s * 512);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         r.w[4 * s + j] = v[j];
@@ -301,14 +282,14 @@ __device__ __forceinline__ void load_slice(SliceRegs<G>& r, const uint8_t* group
   } else {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x2_t v = L::b8(group + words + s * 512);
+      const u32x2_t v = *reinterpret_cast<const u32x2_t*>(group + words + s * 512);
       r.w[2 * s] = v[0];
       r.w[2 * s + 1] = v[1];
     }
   }
-  r.alpha = L::u16(group + scale);
+  r.alpha = u16(group + scale);
   if constexpr (F == PacketFormat::kNativeAsym) {
-    r.beta = L::u16(group + scale + 4);
+    r.beta = u16(group + scale + 4);
   }
 }
 
@@ -498,7 +479,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p
       const int g = min(g0 + wp * KG + kk, p.NG - 1);
 #pragma unroll
       for (int j = 0; j < CS; ++j) {
-        load_slice<G, F, T::kOnce>(w[kk][j], slice0[j] + static_cast<size_t>(g) * kStride, words, scale[j]);
+        load_slice<G, F>(w[kk][j], slice0[j] + static_cast<size_t>(g) * kStride, words, scale[j]);
       }
     }
   };
