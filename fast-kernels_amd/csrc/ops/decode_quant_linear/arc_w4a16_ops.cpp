@@ -892,10 +892,11 @@ bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group
 // Estimated time, in us, of a plan of 16-row tiles: rounds of workgroups, each start-up and groups,
 // and the fix-up of K splits. The lower of two fits. The first, like the row tiles', is to 560 bf16
 // launches over native slabs, in whole rounds (deviation 6-8 %). The second is to 1480 drawn launches of
-// both activation types over all packet formats (9-10 %); runs of up to 3072 values share a CU, so
-// workgroups just past a whole round cost less than another one (39 rows, 11520 x 1920 G128 fp16, 270
-// workgroups: 19.0 us by the first fit, 14.9 measured, the row tiles 17.9). By the first fit alone 13 of
-// the 625 drawn launches on the row tiles were slower there by 3-20 %, by both 8 by up to 11 %.
+// both activation types over all packet formats (9-10 %), for runs of up to 2048 values: several share
+// a CU, so workgroups just past a whole round cost less than another one (39 rows, 11520 x 1920 G128
+// fp16, 270 workgroups: 19.0 us by the first fit, 14.9 measured, the row tiles 17.9). By the first fit
+// alone 13 of the 625 drawn launches on the row tiles were slower there by 3-20 %, by both 10 by up to
+// 11 %.
 double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
   struct Fit {
     double first, per_1024_k, round, round_per_1024_k, fix, short_k;  // short_k: K up to 1024, loaded at once
@@ -912,7 +913,7 @@ double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
            rounds * (c.round + c.round_per_1024_k * kk) +
            (plan.max_tile_contributors > 1 ? c.fix : 0.0);
   };
-  return std::min(us(whole, more), us(shared, kk <= 3 ? (more + over) / 2 : more));
+  return kk > 2 ? us(whole, more) : std::min(us(whole, more), us(shared, (more + over) / 2));
 }
 
 // The row-tile GEMM (w4a16_gemm_tile.hip). plain: no fused neighbour; up to kTileDirectMaxRows rows

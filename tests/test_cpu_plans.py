@@ -21,6 +21,7 @@ def test_workgroups_just_past_a_round_stay_on_16_row_tiles(rows, n, k, g, fmt) -
 @pytest.mark.parametrize("rows,n,k,g,fmt,want", [
     (33, 22016, 4096, 128, 0, 3), (64, 4096, 14336, 128, 1, 3), (512, 10240, 8192, 128, 1, 3),
     (48, 3200, 16064, 64, 0, 3), (46, 13696, 3200, 128, 0, 3), (20, 4096, 14336, 128, 1, 4),
+    (17, 16512, 2112, 64, 0, 4), (64, 8320, 2560, 64, 1, 3),
 ])
 def test_row_tiles_keep_what_they_are_faster_at(rows, n, k, g, fmt, want) -> None:
     assert _schedule(rows, n, k, g, fmt) == want
