@@ -14,7 +14,6 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstdlib>
-#include <limits>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -251,7 +250,7 @@ bool arc_quarter_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_siz
 bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size,
                           int split_k_slices, int cu_count, bool cu_count_given);
 bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
-               int cu_count, double other_us);
+               int cu_count, double limit_us);
 double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count);
 bool is_tile_schedule(int schedule) {
   return schedule == kScheduleTiles || schedule == kScheduleTilesDirect;
@@ -269,7 +268,7 @@ ArcW4A16Plan plan_arc_w4a16_for_cu_count(int batch, int n, int k, int group_size
   }
   if (split_k_slices == 0 && plan.m_tile == fk::kMfmaRows &&
       tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
-                row16_us(plan, group_size, cu_count))) {
+                kTileMargin * row16_us(plan, group_size, cu_count))) {
     return plan;
   }
   if (!arc_stream_plan(plan, batch, n, k, group_size, split_k_slices, cu_count, true)) {
@@ -409,26 +408,66 @@ bool fused_tiles_take(int batch, int n, int k, int group_size, bool silu, int cu
   }
   return batch >= 3 && weights >= (group_size == 64 ? 96LL : 76LL) << 20;
 }
-// What a fused neighbour takes on the dot2 kernels, in us, for tile_plan. From 17 rows: rounds of
-// workgroups of 8 rows and one slice (SiLU: a pair of slices) over all of K, one (G128) or two (G64)
-// per CU. Measured for a round at K 768 / 2048 / 4096, bf16: RMSNorm G128 9.5 / 12.0 / 20, G64 8.4 /
-// 13.3 / 16-21 and 1.3 times that with two workgroups per CU; with SiLU G128 12.2 / 16.3 / 34, G64
-// 10.8 / 20.7 / 37. One round of little K is faster than the row tiles (40 rows, G128: 512 x 1024 9.9
-// and 13.6), two are not (2048 x 1024 18.7 and 14.1).
-double fused_dot2_us(int batch, int n, int k, int group_size, bool silu, int cu_count) {
-  if (batch < kTileMinBatch) {
-    const bool tiles = batch >= 2 && fused_tiles_take(batch, n, k, group_size, silu, cu_count);
-    return tiles ? std::numeric_limits<double>::infinity() : 0.0;
-  }
+// What a fused neighbour of 2-16 rows takes on a dot2 plan, in us: rounds of workgroups, each start-up,
+// its run of K, staged 2048 values at a time, and the fix-up of K splits. Fitted to 2440 drawn launches
+// of both activation types over native slabs (deviation 5-15 %), by the rows of a dot2 tile (2, 4, 8).
+double fused_dot2_small_us(int batch, long long workgroups, int run_k, bool split, int group_size,
+                           bool silu, int cu_count) {
+  struct Fit {
+    double first, per_1024_k, stage, round, round_per_1024_k, fix;
+  };
+  constexpr Fit kNorm64[] = {{4.1, 1.0, 0.9, 0.7, 0.8, 4.7}, {5.5, 1.1, 1.7, 0.7, 1.4, 6.6},
+                             {6.9, 3.2, 1.9, 1.3, 2.2, 8.7}};
+  constexpr Fit kNorm128[] = {{4.2, 0.6, 1.2, 0.9, 0.8, 6.7}, {5.1, 1.2, 1.7, 1.8, 1.3, 7.4},
+                              {7.9, 2.0, 2.8, 3.5, 4.0, 16.8}};
+  constexpr Fit kSilu64[] = {{5.4, 1.5, 2.2, -0.5, 1.9, 0.0}, {7.1, 2.1, 4.3, -1.1, 3.5, 0.0},
+                             {8.5, 6.9, 2.5, 3.0, 3.3, 0.0}};
+  constexpr Fit kSilu128[] = {{5.3, 1.3, 2.2, -0.3, 2.0, 0.0}, {7.2, 1.7, 4.3, 3.2, 4.1, 0.0},
+                              {11.4, 2.8, 8.0, 3.2, 6.4, 0.0}};
+  const int rows = batch <= 2 ? 0 : batch <= 4 ? 1 : 2;
+  const Fit c = group_size == 64 ? (silu ? kSilu64 : kNorm64)[rows] : (silu ? kSilu128 : kNorm128)[rows];
+  const double kk = run_k / 1024.0;
+  const double more = static_cast<double>((workgroups + cu_count - 1) / cu_count - 1);
+  return c.first + c.per_1024_k * kk + c.stage * ((run_k + 2047) / 2048 - 1) +
+         more * (c.round + c.round_per_1024_k * kk) + (split ? c.fix : 0.0);
+}
+// The longest estimate of the row tiles at which a fused neighbour goes to them from its dot2 plan.
+// From 17 rows the dot2 kernels take rounds of workgroups of 8 rows and one slice (SiLU: a pair of
+// slices) over all of K, one (G128) or two (G64) per CU. Measured for a round at K 768 / 2048 / 4096,
+// bf16: RMSNorm G128 9.5 / 12.0 / 20, G64 8.4 / 13.3 / 16-21 and 1.3 times that with two workgroups per
+// CU; with SiLU G128 12.2 / 16.3 / 34, G64 10.8 / 20.7 / 37. One round of little K is faster than the row
+// tiles (40 rows, G128: 512 x 1024 9.9 and 13.6), two are not (2048 x 1024 18.7 and 14.1). Below 17 rows
+// the row tiles, half of them padding, take a * estimate + b * weight MB + c * K / 1024 + d us (716 drawn
+// launches, deviation 4-5 %). By the weights alone 80 of 1431 drawn calls on the row tiles were slower
+// there by more than 3 %, up to twofold (with SiLU, 4 rows, 34816 x 1408 G64: 15.8 and 31.5); with this
+// limit 9 are, by up to 11 %, and 12 that were faster there go back.
+constexpr double kFusedTileMargin = 1.02;
+double fused_tile_limit_us(const ArcW4A16Plan& dot2, int batch, int n, int k, int group_size,
+                           bool silu, int cu_count) {
   const double kk = k / 1024.0;
   const long long slices = (n + fk::kSliceCols - 1) / fk::kSliceCols / (silu ? 2 : 1);
+  if (batch < kTileMinBatch) {
+    if (batch < 2 || !fused_tiles_take(batch, n, k, group_size, silu, cu_count)) {
+      return 0.0;
+    }
+    const long long workgroups =
+        silu ? (batch + dot2.m_tile - 1) / dot2.m_tile * slices : dot2.workgroups;
+    const double us = fused_dot2_small_us(
+        batch, workgroups, dot2.groups_per_workgroup * group_size,
+        dot2.max_tile_contributors > 1, group_size, silu, cu_count);
+    const double weights_mb = 0.5e-6 * n * k;
+    const double rest = group_size == 64 ? 0.091 * weights_mb + 0.31 * kk + 3.7
+                                         : 0.072 * weights_mb + 0.32 * kk + 4.1;
+    return (kFusedTileMargin * us - rest) / (group_size == 64 ? 0.79 : 0.70);
+  }
   const long long workgroups = (batch + 7) / 8 * slices;
   const long long resident = group_size == 64 ? 2LL * cu_count : cu_count;
   const double rounds = static_cast<double>((workgroups + resident - 1) / resident);
   if (group_size == 64) {
-    return rounds * (silu ? 4.8 + 7.9 * kk : (5.5 + 3.9 * kk) * (workgroups > cu_count ? 1.3 : 1.0));
+    return kTileMargin * rounds *
+           (silu ? 4.8 + 7.9 * kk : (5.5 + 3.9 * kk) * (workgroups > cu_count ? 1.3 : 1.0));
   }
-  return rounds * (silu ? 8.8 + 3.8 * kk : 7.6 + 2.3 * kk);
+  return kTileMargin * rounds * (silu ? 8.8 + 3.8 * kk : 7.6 + 2.3 * kk);
 }
 bool mfma_stream_enabled() {
   static const bool enabled = env_enabled("FK_W4A16_MFMA_STREAM");
@@ -919,10 +958,10 @@ double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
 // The row-tile GEMM (w4a16_gemm_tile.hip). plain: no fused neighbour; up to kTileDirectMaxRows rows
 // are then staged by the tiles themselves (kScheduleTilesDirect), without the launch that prepares
 // them. More than kTileMaxRows rows run as several launches over one workspace. False (plan
-// unchanged) when the tiles outnumber the fix-up counters, are not estimated to be faster than another
-// kernel's other_us, or need more workspace than a plain plan of up to 16 rows may.
+// unchanged) when the tiles outnumber the fix-up counters, are estimated to take longer than limit_us,
+// or need more workspace than a plain plan of up to 16 rows may.
 bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
-               int cu_count, double other_us) {
+               int cu_count, double limit_us) {
   const bool direct = tile_direct(batch, plain);
   const int rows = std::min(batch, fk::kTileMaxRows);
   const fk::TileShape s =
@@ -936,7 +975,7 @@ bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool
     us += r.us;
   }
   if (static_cast<std::size_t>(s.mtiles) * s.col_tiles > kMaxFixupCounters ||
-      us > kTileMargin * other_us ||
+      us > limit_us ||
       (plain && batch < kTileMinBatch && bytes > kNoAllocScratchBytes)) {
     return false;
   }
@@ -992,7 +1031,7 @@ ArcW4A16Plan plan_for_format_impl(int batch, int n, int k, int group_size, int a
   if (plain && tiles && split_k_slices == 0 && kernel == kKernelAuto &&
       plan.m_tile == fk::kMfmaRows &&
       tile_plan(plan, batch, n, k, group_size, /*plain=*/true, cu_count,
-                row16_us(plan, group_size, cu_count))) {
+                kTileMargin * row16_us(plan, group_size, cu_count))) {
     return plan;
   }
   if (format == fk::PacketFormat::kArc && plain && kernel != kKernelMfma &&
@@ -2018,15 +2057,15 @@ ArcW4A16Plan silu_mul_plan(int batch, int n, int k, int group_size, int cu_count
   if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/true, cus, given)) {
     return plan;
   }
-  if (with_workspace && tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
-                                  fused_dot2_us(batch, n, k, group_size, /*silu=*/true, cus))) {
-    return plan;
-  }
   plan = ArcW4A16Plan{};
   plan.m_tile = fk::gemv_partials_m_tile_for_batch(batch);
   plan.slice_cols = fk::kSliceCols;
   plan.groups_per_workgroup = k / group_size;
   plan.max_tile_contributors = 1;
+  if (with_workspace) {
+    tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
+              fused_tile_limit_us(plan, batch, n, k, group_size, /*silu=*/true, cus));
+  }
   return plan;
 }
 
@@ -2087,12 +2126,11 @@ ArcW4A16Plan plan_w4a16_fused(int batch, int n, int k, int group_size, int activ
   if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/false, cus, given)) {
     return plan;
   }
-  if (tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
-                fused_dot2_us(batch, n, k, group_size, /*silu=*/false, cus))) {
-    return plan;
-  }
-  return plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, cu_count,
-                              packet_format, kKernelDot2, /*plain=*/false);
+  plan = plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, cu_count, packet_format,
+                              kKernelDot2, /*plain=*/false);
+  tile_plan(plan, batch, n, k, group_size, /*plain=*/false, cus,
+            fused_tile_limit_us(plan, batch, n, k, group_size, /*silu=*/false, cus));
+  return plan;
 }
 
 void w4a16_forward_fused(std::uintptr_t activations_ptr, std::uintptr_t norm_weight_ptr, float eps,

@@ -25,3 +25,25 @@ def test_workgroups_just_past_a_round_stay_on_16_row_tiles(rows, n, k, g, fmt) -
 ])
 def test_row_tiles_keep_what_they_are_faster_at(rows, n, k, g, fmt, want) -> None:
     assert _schedule(rows, n, k, g, fmt) == want
+
+
+def _fused(rows, n, k, g, silu) -> int:
+    return native_module().w4a16_plan_fused(rows, n, k, g, 0, 256, 1, silu)["schedule"]
+
+
+@pytest.mark.parametrize("rows,n,k,g,silu", [
+    (4, 34816, 1408, 64, True), (3, 43776, 1472, 64, True), (5, 7296, 1280, 128, False),
+    (9, 3584, 1280, 128, False), (7, 4736, 1856, 64, False), (5, 4096, 1024, 128, False),
+])
+def test_fused_calls_of_short_k_stay_on_dot2_kernels(rows, n, k, g, silu) -> None:
+    """In us, dot2 and row tiles: 15.8 and 31.5, 21.7 and 32.8, 9.5 and 13.4, 9.7 and 13.0, 12.4 and
+    15.7, 8.3 and 10.9."""
+    assert _fused(rows, n, k, g, silu) == 0
+
+
+@pytest.mark.parametrize("rows,n,k,g,silu", [
+    (13, 32640, 3328, 128, False), (11, 2304, 20160, 64, False), (8, 5760, 2560, 128, False),
+    (5, 1152, 4032, 64, False), (3, 32000, 1664, 128, True), (15, 3584, 1664, 128, True),
+])
+def test_fused_calls_keep_the_row_tiles_where_faster(rows, n, k, g, silu) -> None:
+    assert _fused(rows, n, k, g, silu) == 3
