@@ -71,10 +71,15 @@ WORKLOADS = {
 
 
 # Launch schedules of a plan (fk_arc_w4a16_plan.schedule) and the kernel each runs.
-SCHEDULES = {0: "runs", 1: "slice_pairs", 2: "stream"}
+SCHEDULES = {0: "runs", 1: "slice_pairs", 2: "stream", 3: "row_tiles", 4: "row_tiles_direct"}
 
 
-def kernel_name(packets: str, schedule: int) -> str:
+def kernel_name(packets: str, plan: dict) -> str:
+    schedule = plan.get("schedule", 0)
+    if schedule >= 3:
+        return "w4a16_gemm_tile_kernel"
+    if plan.get("m_tile", 1) == 16:
+        return "w4a16_gemm_mfma_stream_kernel" if schedule == 2 else "w4a16_gemm_mfma_kernel"
     if packets == "arc":
         return "w4a16_gemv_kernel"
     return "w4a16_gemv_stream_kernel" if schedule == 2 else "w4a16_gemv_native_kernel"
@@ -85,10 +90,12 @@ def algorithmic_bytes(batch: int, n: int, k: int, g: int) -> int:
 
 
 def _threads_per_workgroup(plan: dict, num_groups: int) -> int:
-    """Threads of one workgroup: 256 for the per-slice runs, 8 waves for the stream schedule and a
-    ninth (the control wave) when its workgroups also take a piece of a left-over slice."""
-    if plan.get("schedule", 0) != 2:
-        return 256
+    """Threads of one workgroup: 256 for the per-slice runs, 8 waves for the row tiles and the stream
+    schedule, there with a ninth (the control wave) when its workgroups also take a piece of a
+    left-over slice."""
+    schedule = plan.get("schedule", 0)
+    if schedule != 2:
+        return 512 if schedule >= 3 else 256
     return 576 if plan["groups_per_workgroup"] % num_groups else 512
 
 
@@ -522,7 +529,7 @@ def main() -> int:
         "per_shape": per_shape,
         "roofline": {
             "bound": "hbm",
-            "kernel": kernel_name(args.packets, dominant.plan.get("schedule", 0))
+            "kernel": kernel_name(args.packets, dominant.plan)
             + f" ({dominant.name} {dominant.n}x{dominant.k})",
             "achieved": achieved,
             "peak": PEAK_HBM_GBS,

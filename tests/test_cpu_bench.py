@@ -75,3 +75,19 @@ def test_hbm_read_floor_probe_builds_for_gfx950(tmp_path) -> None:
                           capture_output=True, text=True, timeout=600)
     assert proc.returncode == 0, proc.stderr[-2000:]
     assert out.stat().st_size > 0
+
+
+@pytest.mark.parametrize("rows", [1, 4, 8, 16, 17, 33, 512])
+@pytest.mark.parametrize("packets", ["arc", "native"])
+def test_every_schedule_has_a_name_and_a_block(rows: int, packets: str) -> None:
+    """What the JSON line says of a shape's plan, for every workload and the rows --batch takes."""
+    from bench import SCHEDULES, WORKLOADS, _threads_per_workgroup, kernel_name
+    from fast_kernels.native import native_module
+
+    for _, g, shapes in WORKLOADS.values():
+        for _, n, k in shapes:
+            plan = native_module().arc_w4a16_plan(rows, n, k, g, 0, 0, 256, int(packets != "arc"), 0)
+            assert SCHEDULES[plan["schedule"]]
+            tiles = plan["schedule"] in (3, 4)
+            assert (kernel_name(packets, plan) == "w4a16_gemm_tile_kernel") == tiles
+            assert _threads_per_workgroup(plan, k // g) in ((512,) if tiles else (256, 512, 576))
