@@ -1,7 +1,7 @@
 // W4A16 GEMM over row tiles on the gfx950 matrix cores: 8-16 activation rows that the stream kernel
 // does not take, 17 and more (batched serving, chunks of a prompt), over reference packets or native slabs.
 //
-// Above 32 rows, and under a fused neighbour, a first launch (tile_prepare_kernel) writes the
+// Above 32 rows, and under a fused neighbour, a first launch (w4a16_gemm_tile_prepare_kernel) writes the
 // activations in the order the tiles read them: re-paired (x0,x4)(x1,x5)(x2,x6)(x3,x7) like the code
 // words unpack, [32-row block][group][16-byte unit][row], so staging is a straight copy and every
 // LDS access is 512 consecutive bytes per half wave; beside them the (row, group) sums. It applies
@@ -99,7 +99,7 @@ __device__ __forceinline__ int window_slot(int w, bool quarters) {
 // Rows are read along K (a wave a row) and written 128 bytes (8 rows) at a time, through LDS.
 // kNorm: every workgroup first forms 1 / rms of its rows (fp32, the whole row, from L2).
 template <int G, Act A, bool kNorm>
-__global__ void __launch_bounds__(kPrepThreads) tile_prepare_kernel(PrepareParams p) {
+__global__ void __launch_bounds__(kPrepThreads) w4a16_gemm_tile_prepare_kernel(PrepareParams p) {
   constexpr int WR = G / 8;
   __shared__ u32x4_t turn[kPrepUnits * kPrepRows];
   const int tid = static_cast<int>(threadIdx.x);
@@ -238,7 +238,7 @@ struct SliceRegs {
 // Byte offsets of a lane in a group's slab (native) or packet (kArc, of 32-column quarter 0):
 // words of its window 0, and its alpha. Column lane % 32, half h = lane / 32. Native window v
 // holds word U (2 (v / U) + h) + v % U of the group (U = G / 32: the layout's quarter units), kArc
-// word 2 v + h; tile_prepare_kernel orders the activations alike.
+// word 2 v + h; w4a16_gemm_tile_prepare_kernel orders the activations alike.
 template <int G, PacketFormat F>
 __device__ __forceinline__ uint32_t lane_words(int lane) {
   const int c = lane % 32;
@@ -412,7 +412,7 @@ __device__ __forceinline__ bool has_non_finite_bf16(uint32_t pair) {
 // window between the MFMAs. LDS rows are swizzled by the unit's place (consecutive lanes store
 // consecutive units of one row, 512 bytes apart).
 template <class T, Act A, PacketFormat F, bool kSilu, bool kDirect>
-__global__ void __launch_bounds__(kTileThreads, 2) tile_gemm_kernel(TileParams p) {
+__global__ void __launch_bounds__(kTileThreads, 2) w4a16_gemm_tile_kernel(TileParams p) {
   constexpr int G = T::G;
   constexpr int RS = T::RS;
   constexpr int CS = T::CS;
@@ -872,7 +872,7 @@ using Tile128 = Tile<G, 2, 2, 2, 4, 1>;  // 128 x 256
 
 template <class T, Act A, PacketFormat F, bool kSilu, bool kDirect = false>
 hipError_t launch_tile(const TileParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((tile_gemm_kernel<T, A, F, kSilu, kDirect>), dim3(p.grid), dim3(kTileThreads),
+  hipLaunchKernelGGL((w4a16_gemm_tile_kernel<T, A, F, kSilu, kDirect>), dim3(p.grid), dim3(kTileThreads),
                      T::kLdsBytes, stream, p);
   return hipGetLastError();
 }
@@ -918,9 +918,9 @@ hipError_t launch_typed(const TileLaunch& l, const TileShape& s, hipStream_t str
   const dim3 pgrid(static_cast<unsigned int>(s.mtiles * s.bm / kPrepRows),
                    static_cast<unsigned int>((l.K / 8 + kPrepUnits - 1) / kPrepUnits));
   if (l.norm_weight != nullptr) {
-    hipLaunchKernelGGL((tile_prepare_kernel<G, A, true>), pgrid, dim3(kPrepThreads), 0, stream, q);
+    hipLaunchKernelGGL((w4a16_gemm_tile_prepare_kernel<G, A, true>), pgrid, dim3(kPrepThreads), 0, stream, q);
   } else {
-    hipLaunchKernelGGL((tile_prepare_kernel<G, A, false>), pgrid, dim3(kPrepThreads), 0, stream, q);
+    hipLaunchKernelGGL((w4a16_gemm_tile_prepare_kernel<G, A, false>), pgrid, dim3(kPrepThreads), 0, stream, q);
   }
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) {
     return e;

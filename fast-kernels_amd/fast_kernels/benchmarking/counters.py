@@ -63,17 +63,19 @@ def _profile(rocprof: str, counter: str, child_args: list[str], out_dir: Path) -
 
 
 def _kernel_counter(directory: Path, counter: str) -> float | None:
-    """Mean counter value per dispatch of the case's W4A16 kernel (the grid with most dispatches)."""
-    best: tuple[int, float] | None = None
+    """Mean counter value per launch of the case's W4A16 kernel (the grid with most dispatches; the
+    row tiles' prepare launch, dispatched as often as their GEMM, adds its own)."""
+    groups: list[tuple[int, float]] = []
     for name_filter in KERNEL_NAME_FILTERS:
         try:
-            groups = counter_by_grid(directory, counter, name_filter, with_counts=True)
+            found = counter_by_grid(directory, counter, name_filter, with_counts=True)
         except FileNotFoundError:
             return None
-        for _, (mean, count) in groups.items():
-            if best is None or count > best[0]:
-                best = (count, mean)
-    return None if best is None else best[1]
+        groups += [(count, mean) for mean, count in found.values()]
+    if not groups:
+        return None
+    most = max(count for count, _ in groups)
+    return sum(mean for count, mean in groups if count == most)
 
 
 def add_traffic_metrics(suite_path: Path, cases: list[BenchmarkCase]) -> list[str]:

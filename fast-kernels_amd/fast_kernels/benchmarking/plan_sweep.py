@@ -127,7 +127,7 @@ SPLITS = (1, 2, 3, 4, 6, 8, 16)
 KERNELS = {"auto": 0, "dot2": 1, "mfma": 2}
 FORMATS = {"arc": 0, "native_sym": 1, "native_asym": 2}
 PLAN_KEYS = ("m_tile", "workgroups", "groups_per_workgroup", "slice_cols", "schedule")
-SCHEDULE_NAMES = {0: "runs", 1: "pairs", 2: "stream"}
+SCHEDULE_NAMES = {0: "runs", 1: "pairs", 2: "stream", 3: "tiles", 4: "tiles direct"}
 
 
 def _plan_label(plan: dict[str, int]) -> str:

@@ -4,11 +4,13 @@ grid), and the duration split that separates two shapes sharing one kernel and g
 from __future__ import annotations
 
 import csv
+import re
 import sys
 from pathlib import Path
 
 sys.path.insert(0, str(Path(__file__).resolve().parent.parent / "fast-kernels_amd"))
 
+from fast_kernels.benchmarking.counters import _kernel_counter  # noqa: E402
 from fast_kernels.benchmarking.rocprof import kernel_trace_by_grid  # noqa: E402
 
 FIELDS = ["Kind", "Kernel_Name", "Start_Timestamp", "End_Timestamp", "Workgroup_Size_X",
@@ -58,3 +60,33 @@ def test_split_keeps_one_shape_across_the_cut(tmp_path: Path) -> None:
     d = _write(tmp_path / "c", [(KERNEL, 131072, 19900)] * 25 + [(KERNEL, 131072, 20400)] * 75)
     rows = kernel_trace_by_grid(d, "w4a16", split_us=20)
     assert len(rows) == 1 and rows[0]["calls"] == 100
+
+
+def test_the_row_tiles_kernels_are_counted(tmp_path: Path) -> None:
+    """The traffic of a row-tile case is that of its two launches, under the names that the source
+    gives them; other kernels of the process do not count."""
+    source = (Path(__file__).resolve().parent.parent / "fast-kernels_amd" / "csrc" / "kernels" /
+              "decode_quant_linear" / "w4a16_gemm_tile.hip").read_text()
+    kernels = re.findall(r"__global__ void __launch_bounds__\([^)]*\)\s*(\w+)\(", source)
+    assert len(kernels) == 2
+    rows = [(f"void fk::(anonymous namespace)::{name}<128>(P)", 4096 * (i + 1), 100.0 * (i + 1))
+            for i, name in enumerate(kernels) for _ in range(20)]
+    rows += [("void fk::(anonymous namespace)::pack_kernel<128>(P)", 64, 7.0)]
+    rows += [("void fk::(anonymous namespace)::w4a16_gemm_mfma_kernel<128>(P)", 64, 7.0)] * 3
+    with (tmp_path / "x_counter_collection.csv").open("w", newline="") as fh:
+        w = csv.DictWriter(fh, fieldnames=["Counter_Name", "Kernel_Name", "Grid_Size", "Counter_Value"])
+        w.writeheader()
+        for name, grid, value in rows:
+            w.writerow({"Counter_Name": "FETCH_SIZE", "Kernel_Name": name, "Grid_Size": grid,
+                        "Counter_Value": value})
+    assert _kernel_counter(tmp_path, "FETCH_SIZE") == 300.0
+
+
+def test_every_schedule_has_a_sweep_label() -> None:
+    from fast_kernels.benchmarking.plan_sweep import SCHEDULE_NAMES
+    from fast_kernels.native import native_module
+
+    plans = [native_module().arc_w4a16_plan(m, 4096, 14336, 128, 0, 0, 256, 1, 0)
+             for m in (1, 4, 20, 64)]
+    assert {p["schedule"] for p in plans} >= {3, 4}
+    assert all(p["schedule"] in SCHEDULE_NAMES for p in plans)
