@@ -339,47 +339,72 @@ __device__ __forceinline__ uint32_t silu_mul_pair(uint32_t gw, uint32_t uw) {
   return o;
 }
 
-// One output in plain fp32 arithmetic on activations 2^-64 times smaller: for bf16 outputs that
-// came out infinite or NaN. The tile's accumulators hold sums of (128 + q) x, which overflow from
-// |x| of about 2^113; the result itself may still be finite.
+// The activations of unit w of group g of a row, paired (values i and i + 4).
 template <int G, PacketFormat F, bool kDirect>
-__device__ __forceinline__ uint16_t plain_bf16_output(const TileParams& p, int row, int col) {
+__device__ __forceinline__ u32x4_t paired_unit(const TileParams& p, int row, int g, int w) {
   constexpr int WR = G / 8;
+  if constexpr (kDirect) {
+    const u32x4_t v =
+        reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(row) * p.K)[g * WR + w];
+    const uint4 q = pair_activations(make_uint4(v.x, v.y, v.z, v.w));
+    return u32x4_t{q.x, q.y, q.z, q.w};
+  } else {
+    const u32x4_t* xr =
+        p.xs + static_cast<size_t>(row / kBlockRows) * p.NG * (WR * kBlockRows) + row % kBlockRows;
+    return xr[(g * WR + window_slot<G>(w, is_native(F))) * kBlockRows];
+  }
+}
+
+__device__ __forceinline__ bool has_non_finite_bf16(uint32_t pair) {
+  return (pair & 0x7f80u) == 0x7f80u || (pair & 0x7f800000u) == 0x7f800000u;
+}
+
+// Whether a row of bf16 activations holds neither infinities nor NaN (asked by a whole wave).
+template <int G, PacketFormat F, bool kDirect>
+__device__ bool finite_row(const TileParams& p, int row, int lane) {
+  constexpr int WR = G / 8;
+  bool bad = false;
+#pragma unroll 4
+  for (int u = lane; u < p.NG * WR; u += 64) {
+    const u32x4_t x = paired_unit<G, F, kDirect>(p, row, u / WR, u % WR);
+    bad |= has_non_finite_bf16(x[0]) || has_non_finite_bf16(x[1]) || has_non_finite_bf16(x[2]) ||
+           has_non_finite_bf16(x[3]);
+  }
+  return !__any(bad);
+}
+
+// One output in plain fp32 arithmetic on activations 2^-64 times smaller, by a whole wave: for bf16
+// outputs that came out infinite or NaN from finite activations. The tile's accumulators hold sums of
+// (128 + q) x, which overflow from |x| of about 2^113; the result itself may still be finite. (By one
+// lane an output, and for rows that hold a NaN too, one such row of 64, 28672 x 4096, made a call of 28
+// us take 1556; now 32.)
+template <int G, PacketFormat F, bool kDirect>
+__device__ uint16_t plain_bf16_output(const TileParams& p, int row, int col, int lane) {
+  constexpr int WR = G / 8;
+  constexpr int U = native_unit_words(G);
   constexpr int kStride = format_packet_stride(G, F);
   const uint8_t* base =
       p.packets + static_cast<size_t>(is_native(F) ? col / kSliceCols : col / kTileCols) * p.NG * kStride;
   const int c = is_native(F) ? col % kSliceCols : col % kTileCols;
-  const u32x4_t* xr =
-      kDirect ? reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(row) * p.K)
-              : p.xs + static_cast<size_t>(row / kBlockRows) * p.NG * (WR * kBlockRows) + row % kBlockRows;
   float y = 0.0f;
-#pragma unroll 1
-  for (int g = 0; g < p.NG; ++g) {
+#pragma unroll 2
+  for (int u = lane; u < p.NG * WR; u += 64) {
+    const int g = u / WR;
+    const int w = u % WR;
     const uint8_t* group = base + static_cast<size_t>(g) * kStride;
+    const u32x4_t x = paired_unit<G, F, kDirect>(p, row, g, w);
+    const int at = is_native(F) ? native_word_offset(G, c / 16, w / U, c % 16, w % U)
+                                : (w * kTileCols + c) * 4;
+    const uint32_t word = *reinterpret_cast<const uint32_t*>(group + at);
     float dot = 0.0f;
     float sum = 0.0f;
-#pragma unroll 1
-    for (int w = 0; w < WR; ++w) {
-      u32x4_t x;  // paired: values i and i + 4
-      if constexpr (kDirect) {
-        const u32x4_t v = xr[g * WR + w];
-        const uint4 q = pair_activations(make_uint4(v.x, v.y, v.z, v.w));
-        x = u32x4_t{q.x, q.y, q.z, q.w};
-      } else {
-        x = xr[(g * WR + window_slot<G>(w, is_native(F))) * kBlockRows];
-      }
-      constexpr int U = native_unit_words(G);
-      const int at = is_native(F) ? native_word_offset(G, c / 16, w / U, c % 16, w % U)
-                                  : (w * kTileCols + c) * 4;
-      const uint32_t word = *reinterpret_cast<const uint32_t*>(group + at);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float lo = bf16_bits_to_float(static_cast<uint16_t>(x[i])) * 0x1p-64f;
-        const float hi = bf16_bits_to_float(static_cast<uint16_t>(x[i] >> 16)) * 0x1p-64f;
-        dot = fmaf(static_cast<float>((word >> (4 * i)) & 15u), lo, dot);
-        dot = fmaf(static_cast<float>((word >> (4 * i + 16)) & 15u), hi, dot);
-        sum += lo + hi;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const float lo = bf16_bits_to_float(static_cast<uint16_t>(x[i])) * 0x1p-64f;
+      const float hi = bf16_bits_to_float(static_cast<uint16_t>(x[i] >> 16)) * 0x1p-64f;
+      dot = fmaf(static_cast<float>((word >> (4 * i)) & 15u), lo, dot);
+      dot = fmaf(static_cast<float>((word >> (4 * i + 16)) & 15u), hi, dot);
+      sum += lo + hi;
     }
     uint16_t a_bits = 0;
     float beta = 0.0f;
@@ -400,11 +425,11 @@ __device__ __forceinline__ uint16_t plain_bf16_output(const TileParams& p, int r
     y = fmaf(half_bits_to_float(a_bits), dot, y);
     y = fmaf(beta, sum, y);
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    y += __shfl_xor(y, off);
+  }
   return float_to_bf16_bits(y * 0x1p64f);
-}
-
-__device__ __forceinline__ bool has_non_finite_bf16(uint32_t pair) {
-  return (pair & 0x7f80u) == 0x7f80u || (pair & 0x7f800000u) == 0x7f800000u;
 }
 
 // kDirect: the workgroup stages the activations itself, from x, instead of copying prepared ones: a
@@ -819,24 +844,41 @@ __global__ void __launch_bounds__(kTileThreads, 2) w4a16_gemm_tile_kernel(TilePa
   const int out_n = kSilu ? p.N / 2 : p.N;
   constexpr int kCols = kSilu ? T::kBN / 2 : T::kBN;
   const int col0 = ct * kCols;
+  int asked_row = -1;  // the last row that finite_row was asked about, and its answer
+  bool asked_finite = false;
+  static_assert(T::kBM * (kCols / 8) % 64 == 0, "whole waves");
   for (int e = tid; e < T::kBM * (kCols / 8); e += kTileThreads) {
     const int row = e / (kCols / 8);
     const int c = e % (kCols / 8) * 8;
-    if (row0 + row >= p.M || col0 + c >= out_n) {
-      continue;
-    }
+    const bool live = row0 + row < p.M && col0 + c < out_n;
     auto outputs = [&](int tile_col, int col) {
       u32x4_t o = *reinterpret_cast<const u32x4_t*>(tile16 + row * T::kOutPitch + tile_col);
       if constexpr (A == Act::kBF16) {
-        if (has_non_finite_bf16(o[0]) || has_non_finite_bf16(o[1]) || has_non_finite_bf16(o[2]) ||
-            has_non_finite_bf16(o[3])) {
+        const bool bad = live && (has_non_finite_bf16(o[0]) || has_non_finite_bf16(o[1]) ||
+                                  has_non_finite_bf16(o[2]) || has_non_finite_bf16(o[3]));
+        // by the whole wave, one lane's outputs after another's
+        for (uint64_t todo = __ballot(bad); todo != 0; todo &= todo - 1) {
+          const int of = __builtin_ctzll(todo);
+          const int of_row = __builtin_amdgcn_readlane(row, of);
+          const int of_col = __builtin_amdgcn_readlane(col, of);
+          uint16_t* at = tile16 + of_row * T::kOutPitch + __builtin_amdgcn_readlane(tile_col, of);
+          if (of_row != asked_row) {
+            asked_row = of_row;
+            asked_finite = finite_row<G, F, kDirect>(p, row0 + of_row, lane);
+          }
+          if (!asked_finite) {
+            continue;
+          }
 #pragma unroll 1
           for (int q = 0; q < 8; ++q) {
-            uint16_t* at = tile16 + row * T::kOutPitch + tile_col + q;
-            if ((*at & 0x7f80u) == 0x7f80u) {
-              *at = plain_bf16_output<G, F, kDirect>(p, row0 + row, col + q);
+            if ((at[q] & 0x7f80u) == 0x7f80u) {
+              at[q] = plain_bf16_output<G, F, kDirect>(p, row0 + of_row, of_col + q, lane);
             }
           }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (bad) {
           o = *reinterpret_cast<const u32x4_t*>(tile16 + row * T::kOutPitch + tile_col);
         }
       }
@@ -849,6 +891,9 @@ __global__ void __launch_bounds__(kTileThreads, 2) w4a16_gemm_tile_kernel(TilePa
       for (int q = 0; q < 4; ++q) {
         o[q] = silu_mul_pair<A>(o[q], up[q]);
       }
+    }
+    if (!live) {
+      continue;
     }
     uint16_t* dst = p.out + static_cast<size_t>(row0 + row) * out_n + col0 + c;
     if (p.vector_out) {

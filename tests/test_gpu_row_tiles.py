@@ -146,3 +146,33 @@ def test_row_tiles_at_the_ends_of_bf16(rows, n, groups, exponent, fmt) -> None:
     assert not torch.isfinite(again[3]).any()
     keep = [r for r in range(rows) if r != 3]
     assert torch.equal(again[keep], got[keep])
+
+
+@pytest.mark.parametrize("rows", [32, 64, 512])
+@pytest.mark.parametrize("value", [math.nan, math.inf])
+def test_a_non_finite_row_costs_little(rows, value) -> None:
+    """A row that holds a NaN (a padded one, say) leaves a bf16 call's time as it is: nothing is
+    computed again for it. At most three times, for the clock's sake; again by one lane an output it
+    would be fifty times and more."""
+    n, k = 28672, 4096
+    case = make_case(1, 128, k, 128, act="bf16", seed=1)
+    x = torch.randn((rows, k), device="cuda").to(torch.bfloat16)
+    packets = _packets(case, "native_sym").repeat(n // 128, 1)
+    case.n = n
+    bad = x.clone()
+    bad[rows // 2, 5] = value
+    times = []
+    for inputs in (x, bad, x, bad):
+        _forward(case, inputs, packets, "native_sym")
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(10):
+            out = _forward(case, inputs, packets, "native_sym")
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 100.0)
+    print("us a call:", [round(t, 1) for t in times])
+    assert min(times[1], times[3]) <= 3 * min(times[0], times[2])
+    assert not torch.isfinite(out[rows // 2]).any()
+    rest = [r for r in range(rows) if r != rows // 2]
+    assert torch.equal(out[rest], _forward(case, x, packets, "native_sym")[rest])
