@@ -115,6 +115,14 @@ PYBIND11_MODULE(_native, m) {
       py::arg("activations_ptr"), py::arg("packets_ptr"), py::arg("group_sums_ptr"),
       py::arg("output_ptr"), py::arg("batch"), py::arg("n"), py::arg("k"), py::arg("group_size"),
       py::arg("packet_stride_bytes"), py::arg("stream_ptr"));
+  m.def(
+      "stream_capture_id",
+      [](std::uintptr_t stream_ptr) {
+        unsigned long long id = 0;
+        check(fk_w4a16_stream_capture_id(mp(stream_ptr), &id));
+        return id;
+      },
+      py::arg("stream_ptr"));
   m.def("release_workspaces", [] { call([] { return fk_w4a16_release_workspaces(); }); });
   m.def(
       "arc_w4a16_forward_split_k",

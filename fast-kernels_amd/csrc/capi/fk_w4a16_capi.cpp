@@ -70,6 +70,15 @@ int fk_arc_w4a16_forward(const void* activations, const void* packets, const voi
   });
 }
 
+int fk_w4a16_stream_capture_id(void* stream, unsigned long long* id) {
+  return guarded([&] {
+    if (id == nullptr) {
+      throw std::invalid_argument("id must not be null");
+    }
+    *id = ops::stream_capture_id(P(stream));
+  });
+}
+
 int fk_w4a16_release_workspaces(void) {
   return guarded([] { ops::release_workspaces(); });
 }

@@ -52,6 +52,12 @@ int fk_arc_w4a16_forward(const void* activations, const void* packets, const voi
   return FK_ERR_RUNTIME;
 }
 
+int fk_w4a16_stream_capture_id(void* stream, unsigned long long* id) {
+  (void)stream;
+  (void)id;
+  return FK_ERR_RUNTIME;
+}
+
 int fk_w4a16_release_workspaces(void) { return FK_ERR_RUNTIME; }
 
 int fk_arc_w4a16_forward_split_k(const void* activations, const void* packets, const void* group_sums, void* partials, int batch, int n, int k, int group_size, int packet_stride_bytes, int split_k_slices, void* stream) {

@@ -27,6 +27,9 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
                        std::uintptr_t group_sums_ptr, std::uintptr_t output_ptr, int batch, int n,
                        int k, int group_size, int packet_stride_bytes, std::uintptr_t stream_ptr);
 
+// The capture under way on a stream (a number of its own for each), 0 for none.
+unsigned long long stream_capture_id(std::uintptr_t stream_ptr);
+
 // Frees what arc_w4a16_forward keeps for calls of many rows (prepared activations and partial tiles:
 // up to 96 MB for each of the last eight streams); the next such call allocates again.
 void release_workspaces();

@@ -1655,6 +1655,14 @@ void arc_w4a16_forward(std::uintptr_t activations_ptr, std::uintptr_t packets_pt
            kActivationF16, stream);
 }
 
+unsigned long long stream_capture_id(std::uintptr_t stream_ptr) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  check_hip(hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>(stream_ptr), &status, &id),
+            "hipStreamGetCaptureInfo");
+  return status == hipStreamCaptureStatusNone ? 0 : id;
+}
+
 void release_workspaces() {
   LibraryMemory& memory = library_memory();
   const std::lock_guard<std::mutex> lock(memory.mutex);

@@ -34,7 +34,8 @@ except ImportError:  # pragma: no cover - every op then raises RuntimeError
 if TYPE_CHECKING:  # pragma: no cover
     import torch
 
-_ARC_WORKSPACE_CACHE: dict[tuple[int, int], Any] = {}
+# (device, stream, whether captured) -> (capture or 0, workspace)
+_ARC_WORKSPACE_CACHE: dict[tuple[int, int, bool], tuple[int, Any]] = {}
 _ARC_SPLIT_K_PARTIALS_CACHE: dict[tuple[int, int, int, int], Any] = {}
 _ARC_WEIGHT_BUFFER_CACHE: dict[tuple[int, int, int], Any] = {}
 _ARC_VENDOR_WORKSPACE_CACHE: dict[tuple[int, int], Any] = {}
@@ -212,15 +213,19 @@ def arc_workspace(device: Any, nbytes: int) -> Any:
     """Zero-filled uint8 workspace of at least nbytes for (device, current stream), cached.
 
     The GEMV's split-K counters return to zero after every launch, so the buffer stays valid for
-    later calls on the same stream. Calls on different streams get different buffers.
+    later calls on the same stream. Calls on different streams get different buffers. The captured
+    calls of a graph share one from the graph's own memory, zero-filled by the graph: an eager call
+    that needs a larger one does not free it, and a graph does not rely on another one's fill.
     """
     torch = _require_torch()
-    key = (_device_index(device), _current_stream_ptr(device))
-    ws = _ARC_WORKSPACE_CACHE.get(key)
-    if ws is None or ws.numel() < nbytes:
+    stream = _current_stream_ptr(device)
+    capture = native_module().stream_capture_id(stream)
+    key = (_device_index(device), stream, capture != 0)
+    held, ws = _ARC_WORKSPACE_CACHE.get(key, (0, None))
+    if ws is None or held != capture or ws.numel() < nbytes:
         size = max(int(nbytes), 1 << 20)
         ws = torch.zeros(size, device=device, dtype=torch.uint8)
-        _ARC_WORKSPACE_CACHE[key] = ws
+        _ARC_WORKSPACE_CACHE[key] = (capture, ws)
     return ws
 
 

@@ -68,6 +68,10 @@ int fk_arc_w4a16_forward(const void* activations, const void* packets, const voi
                          void* output, int batch, int n, int k, int group_size,
                          int packet_stride_bytes, void* stream);
 
+/* Number of the graph capture under way on a stream, 0 for none: a caller that keeps workspaces per
+ * stream takes one of the capture's own, which no eager call replaces or frees. */
+int fk_w4a16_stream_capture_id(void* stream, unsigned long long* id);
+
 /* Frees what fk_arc_w4a16_forward holds for eager calls of many rows; the next one allocates again. */
 int fk_w4a16_release_workspaces(void);
 
