@@ -64,6 +64,22 @@ def _check(case, y: torch.Tensor, cols: np.ndarray) -> None:
     assert np.all(err <= bar), f"max error {err.max():.4g}"
 
 
+def _check_all(case, y: torch.Tensor) -> None:
+    """Every output against the 64-bit product of the dequantised weight: half an ulp of the output, and
+    the fp32 sums' own error. Those sums run over (64 or 128 + q) x, at most 143 |x| alpha_max a term, and
+    round once per 16 terms within a group and once per group, each by 2^-24 of a partial sum that is
+    at most the row's 143 alpha_max sum |x|; 16 of them at full size cover what random signs leave."""
+    codes = torch.from_numpy(case.q_u8).cuda()
+    codes = torch.stack((codes & 15, codes >> 4), dim=-1).view(case.n, -1, case.group_size)
+    alpha, beta = (_tensor(t, torch.float16).double() for t in (case.alpha, case.beta))
+    x = _tensor(case.x, DTYPES[case.act]).double()
+    want = x @ (codes.double() * alpha[..., None] + beta[..., None]).view(case.n, case.k).t()
+    ulp = 2.0**-11 if case.act == "f16" else 2.0**-8
+    sums = 16 * 2.0**-24 * 143 * alpha.max() * x.abs().sum(dim=1, keepdim=True)
+    err = (y.double() - want).abs()
+    assert torch.all(err <= ulp * want.abs() * (1 + 2.0**-6) + sums), f"max error {err.max():.4g}"
+
+
 # rows, columns, groups by group size, then (m_tile, K split): edges of the tiles (32, 64, 128 rows; 128
 # and 256 columns; units of 8 or 16 groups) and one group, among shapes the 16-row tiles are slower
 # at; more rows than one launch takes
@@ -100,6 +116,29 @@ def test_row_tiles_match_oracle(rows, n, groups, group_size, want, act, fmt) -> 
     torch.cuda.synchronize()
     assert torch.equal(y, odd)
     _check(case, y, np.unique(np.linspace(0, n - 1, min(n, 96)).astype(int)))
+    _check_all(case, y)
+
+
+def test_row_tiles_on_two_streams_at_once() -> None:
+    """Calls with K splits on two streams whose launches overlap: neither shares counters or partial
+    tiles with the other (both schedules)."""
+    runs = []
+    for rows, n, groups in ((20, 4096, 112), (96, 3200, 33)):
+        case = make_case(rows, n, groups * 128, 128, act="bf16", seed=rows)
+        x, packets = _tensor(case.x, torch.bfloat16), _packets(case, "native_sym")
+        runs.append((case, x, packets, _forward(case, x, packets, "native_sym")))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        outs = [[], []]
+        for _ in range(10):
+            for i, stream in enumerate(streams):
+                with torch.cuda.stream(stream):
+                    for case, x, packets, _ in runs[:: 1 if i else -1]:
+                        outs[i].append((case.batch, _forward(case, x, packets, "native_sym")))
+        torch.cuda.synchronize()
+        want = {case.batch: y for case, _, _, y in runs}
+        assert all(torch.equal(y, want[m]) for got in outs for m, y in got)
 
 
 @pytest.mark.parametrize("rows,n,groups", [(20, 256, 64), (96, 3200, 33)])
