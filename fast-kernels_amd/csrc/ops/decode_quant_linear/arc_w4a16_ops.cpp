@@ -2131,7 +2131,12 @@ ArcW4A16Plan plan_w4a16_fused(int batch, int n, int k, int group_size, int activ
   }
   const bool given = cu_count > 0;
   const int cus = given ? cu_count : device_cu_count();
-  if (fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/false, cus, given)) {
+  // Two bf16 rows of one dot2 staging chunk, at most a slice per CU: what the matrix cores save does not
+  // pay for their staging (RMSNorm + 2048 / 8192 x 2048 G128 5.5 / 5.8 us on dot2, 6.0 / 6.5 there; fp16,
+  // staged as it is, 5.1 / 5.5 and 4.9 / 5.4; 24576 x 2048 bf16 11.3 and 9.2).
+  const bool dot2_pays = activation_dtype == kActivationBF16 && batch == 2 && k <= 2048 &&
+                         n / fk::kSliceCols <= cus;
+  if (!dot2_pays && fused_mfma_plan(plan, batch, n, k, group_size, /*silu=*/false, cus, given)) {
     return plan;
   }
   plan = plan_for_format_impl(batch, n, k, group_size, activation_dtype, 0, cu_count, packet_format,

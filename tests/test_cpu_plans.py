@@ -47,3 +47,13 @@ def test_fused_calls_of_short_k_stay_on_dot2_kernels(rows, n, k, g, silu) -> Non
 ])
 def test_fused_calls_keep_the_row_tiles_where_faster(rows, n, k, g, silu) -> None:
     assert _fused(rows, n, k, g, silu) == 3
+
+
+@pytest.mark.parametrize("act,n,k,want", [
+    (1, 2048, 2048, 0), (1, 8192, 2048, 0), (0, 8192, 2048, 2), (1, 24576, 2048, 2), (1, 2048, 4096, 2),
+])
+def test_two_bf16_rows_of_short_k_stay_on_dot2(act, n, k, want) -> None:
+    """RMSNorm at 2 rows, dot2 and matrix cores in us: 5.5 and 6.0, 5.8 and 6.5; fp16 5.5 and 5.4; one
+    and a half slices per CU 11.3 and 9.2."""
+    plan = native_module().w4a16_plan_fused(2, n, k, 128, act, 256, 1, False)
+    assert plan["schedule"] == want
