@@ -21,8 +21,8 @@ hipError_t launch_reduce_partials(const void* partials, void* out, int batch, in
 
 // Native packet formats (PacketFormat): build from q_u8 / alpha / zero points (uint8 [N, NG],
 // ignored for kNativeSym), and convert to and from reference packets. arc -> native sets
-// *bad_flag (device uint32, zeroed by the caller) when some beta is not half_rn(-alpha * zp)
-// for an integer zp in 0..15 (zp = 8 for kNativeSym).
+// *bad_flag (a uint32 the GPU can store to, zeroed by the caller; in host memory, with a system-scope
+// store) when some beta is not half_rn(-alpha * zp) for an integer zp in 0..15 (zp = 8 for kNativeSym).
 hipError_t launch_pack_native(const void* q, const void* alpha, const void* zero_points,
                               void* packets, int n, int k, int group_size, PacketFormat format,
                               hipStream_t stream);

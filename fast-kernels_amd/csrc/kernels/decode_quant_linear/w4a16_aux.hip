@@ -59,8 +59,8 @@ dequant_kernel(const uint32_t* __restrict__ q, const uint16_t* __restrict__ alph
 // dequant_arc_packets_kernel (arc_w4a16.cu:183-220): packets -> W[N, K] fp16. A workgroup takes a
 // tile over 256 values of K: 512-byte word rows in, through LDS, 512 bytes of each row of W out
 // (a row's words are 512 bytes apart in the packets: reading them in W's order fetched every line
-// many times over). HBM-bound: 8192 x 8192 G128 69.3 -> 29.6 us back to back (5.8 TB/s; a large copy
-// runs at 5.2), 28672 x 4096 117.5 -> 54.8.
+// many times over). HBM-bound: 8192 x 8192 G128 69.0 -> 27.9 us a call among others (6.1 TB/s; a large
+// copy runs at 5.2), 28672 x 4096 117.5 -> 54.8.
 template <int G>
 __global__ void __launch_bounds__(kAuxThreads)
 dequant_packets_kernel(const uint8_t* __restrict__ packets, uint4* __restrict__ out, int k,

@@ -31,9 +31,10 @@
 //    TFLOP/s over the loop at 8192 x 8192, 512 rows).
 //
 // Measured on MI355X against the 16-row tiles of w4a16_gemm_mfma.hip, which read and unpack the
-// weights once per 16 rows: 10240 x 8192, 512 rows, bf16 native 257 -> 109 us; 4096 x 14336, 64
-// rows 32.0 -> 25.1; 22016 x 4096, 33 rows, fp16 reference packets 35.9 -> 26.5. Of the last two
-// 4-5 us are the first launch and 5-6 the fix-up.
+// weights once per 16 rows: 10240 x 8192, 512 rows, bf16 native 256 -> 108 us; 4096 x 14336, 64
+// rows 31.5 -> 23.5; 22016 x 4096, 33 rows, fp16 reference packets 34.8 -> 25.1. Of the last two
+// about 5 us are the first launch; the 64-row one's seven K splits then meet in the fix-up, the 33-row
+// one's 172 workgroups, one tile each, leave 84 CUs idle.
 #include "w4a16_gemm_tile.h"
 
 #include <cstdint>
@@ -497,7 +498,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) w4a16_gemm_tile_kernel(TilePa
   SliceRegs<G> wreg[2][KG][CS];
   u32x4_t xreg[T::kXPer];
   u32x4_t sreg;
-  // Past the workgroup's last unit (!real): a group that it has just read.
+  // (past the last group, in a short last unit: that group again)
   auto load_weights = [&](int g0, SliceRegs<G> (&w)[KG][CS]) {
 #pragma unroll
     for (int kk = 0; kk < KG; ++kk) {
@@ -618,7 +619,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) w4a16_gemm_tile_kernel(TilePa
   }
   const u32x4_t* s_lane = lds + T::kXUnits + (wp * KG * T::kBlocks + wr * RS) * kBlockRows + (lane & 31);
   for (int u = u_begin; u < u_end; ++u) {
-    // Past the last unit the loads read group 0, which is in the L2.
+    // Past the last unit the loads read group 0, in bounds and used by nobody.
     const int g_next = u + 1 < u_end ? (u + 1) * T::kUnitGroups : 0;
     float b_eff[CS];  // half 0: a pair's even group, half 1: its odd one
     u32x4_t sums[RS];
@@ -1004,7 +1005,10 @@ hipError_t launch_format(const TileLaunch& l, const TileShape& s, hipStream_t st
 
 // Tile choice and K splits by a cost model of the launch, in us, fitted to 560 measured launches (17
 // to 512 rows, 512 to 16384 columns, K from 512 to 6144, bf16 native slabs, MI355X; the fit's
-// standard deviation is 4-8 %): workgroups run one per CU, in rounds of start-up and end (first
+// standard deviation is 4-8 %). Over 645 drawn launches of both types and all formats, to 57344 columns
+// and K of 28672, it is 5 %, 5 % and 0.5 % above the measured times of the 32-, 64- and 128-row tile (its
+// costs are those of non-temporal weight loads, which the first two no longer use), with a standard
+// deviation of 6-8 %, and beyond the fitted sizes within 2 %, 9 % and 2 %: workgroups run one per CU, in rounds of start-up and end (first
 // loads; wave groups' sums, output), units and, with K split, the fix-up (partials out, counter,
 // partials in); `prepare` is the launch before them.
 struct TileCost {

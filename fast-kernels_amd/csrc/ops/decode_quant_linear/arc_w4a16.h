@@ -100,9 +100,9 @@ struct ArcW4A16Plan {
 // slices at once (slice_cols 64); kScheduleStream: one-row native plans on a persistent grid,
 // each workgroup streaming one contiguous range of slabs across slices with the whole activation
 // row staged in LDS (w4a16_gemv_stream.hip).
-// kScheduleTiles: 33 rows and more on the row-tile GEMM (w4a16_gemm_tile.hip): m_tile x slice_cols
-// tiles, K in max_tile_contributors splits; kScheduleTilesDirect: 8 to 32 rows, staged by the
-// tiles, without a launch that prepares them.
+// kScheduleTiles: 33 plain rows and more, and fused neighbours from 2 rows, on the row-tile GEMM
+// (w4a16_gemm_tile.hip): m_tile x slice_cols tiles, K in max_tile_contributors splits;
+// kScheduleTilesDirect: 8 to 32 plain rows, staged by the tiles, without a launch that prepares them.
 enum Schedule : int {
   kScheduleRuns = 0,
   kSchedulePairs = 1,
@@ -179,7 +179,7 @@ void pack_native_w4a16_packets(std::uintptr_t q_ptr, std::uintptr_t alpha_ptr,
 
 // Reference packets -> native packets. Every beta must be half_rn(-alpha * zp) for an integer
 // zp in 0..15 (zp = 8 for the symmetric format), otherwise std::invalid_argument. Synchronises
-// the stream (the check reads a device flag back).
+// the stream (the check reads a flag in host memory that the kernel stores to).
 void convert_arc_w4a16_packets_to_native(std::uintptr_t arc_packets_ptr,
                                          std::uintptr_t native_packets_ptr, int n, int k,
                                          int group_size, int packet_format,
@@ -215,7 +215,8 @@ void w4a16_forward_kernel(std::uintptr_t activations_ptr, std::uintptr_t packets
                           int packet_format, int activation_dtype, int split_k_slices, int kernel,
                           std::uintptr_t stream_ptr);
 
-// arc_w4a16_forward_native (automatic plan) with no workspace argument and no allocation: the
+// arc_w4a16_forward_native with no workspace argument and no allocation: the automatic plan without
+// the row tiles (whose sums run in another order, so that results may differ in their last bit). The
 // fix-up scratch is a fixed per-device array (w4a16_scratch.hip), so launches whose plan needs
 // more than kNoAllocScratchBytes are rejected (std::invalid_argument), and calls that overlap on
 // one device race on it.

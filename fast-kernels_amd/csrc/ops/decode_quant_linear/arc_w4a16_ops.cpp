@@ -382,7 +382,7 @@ constexpr int kMfmaPiecesMinBatch = 3;
 constexpr int kMfmaPiecesMaxBatch = 8;
 // Fused neighbours on the matrix-core stream kernel (us on MI355X, bf16 G128, dot2 runs -> this):
 // RMSNorm + 6144 x 4096 at 2 / 4 / 8 / 16 rows 8.8 -> 7.6, 12.7 -> 7.7, 20.5 -> 10.1, 38.3 -> 14.0;
-// RMSNorm + 28672 x 4096 + SiLU 21.5 -> 16.0, 38.6 -> 16.9, 65.6 -> 19.8, 128.9 -> 24.5. With fewer
+// RMSNorm + 28672 x 4096 + SiLU 21.5 -> 16.0, 38.6 -> 16.9, 65.6 -> 19.8, 128.2 -> 22.7. With fewer
 // than 64 slices only where the dot2 kernels' 8-row tiles are half empty or more than one: RMSNorm +
 // 1024 x 2048 at 2-4 rows 5.4-7.5 either way, at 8 rows 12.0 -> 8.5, at 16 rows 12.1 -> 12.4 (not
 // taken).
@@ -933,9 +933,9 @@ bool arc_mfma_stream_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group
 // launches over native slabs, in whole rounds (deviation 6-8 %). The second is to 1480 drawn launches of
 // both activation types over all packet formats (9-10 %), for runs of up to 2048 values: several share
 // a CU, so workgroups just past a whole round cost less than another one (39 rows, 11520 x 1920 G128
-// fp16, 270 workgroups: 19.0 us by the first fit, 14.9 measured, the row tiles 17.9). By the first fit
-// alone 13 of the 625 drawn launches on the row tiles were slower there by 3-20 %, by both 10 by up to
-// 11 %.
+// fp16, 270 workgroups: 19.0 us by the first fit, 14.9 measured, the row tiles 17.9). Of 1755
+// drawn launches that both send to the row tiles 16 are slower there, by 6-25 %, most of them of several
+// rounds of short runs; longer limits for the second fit cost more gains than that.
 double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
   struct Fit {
     double first, per_1024_k, round, round_per_1024_k, fix, short_k;  // short_k: K up to 1024, loaded at once
@@ -959,7 +959,8 @@ double row16_us(const ArcW4A16Plan& plan, int group_size, int cu_count) {
 // are then staged by the tiles themselves (kScheduleTilesDirect), without the launch that prepares
 // them. More than kTileMaxRows rows run as several launches over one workspace. False (plan
 // unchanged) when the tiles outnumber the fix-up counters, are estimated to take longer than limit_us,
-// or need more workspace than a plain plan of up to 16 rows may.
+// or need more workspace, for up to 16 plain rows, than kNoAllocScratchBytes: automatic plans of those
+// rows are promised to stay within it, whoever brings the memory.
 bool tile_plan(ArcW4A16Plan& plan, int batch, int n, int k, int group_size, bool plain,
                int cu_count, double limit_us) {
   const bool direct = tile_direct(batch, plain);

@@ -138,10 +138,9 @@ typedef struct fk_arc_w4a16_plan {
 #define FK_SCHEDULE_PAIRS 1
 #define FK_SCHEDULE_STREAM 2
 /* FK_SCHEDULE_TILES: 33 rows and more, and fused neighbours of 2 and more, on the row-tile GEMM where
- * that is estimated to be the fastest. m_tile x slice_cols is a workgroup's
- * tile, max_tile_contributors the K splits; the workspace holds the activations as the tiles read
- * them (of up to 1024 rows at a time) besides the counters and partial tiles, and need not be
- * zero-filled. */
+ * that is estimated to be the fastest. m_tile x slice_cols is a workgroup's tile,
+ * max_tile_contributors the K splits; the workspace holds the activations as the tiles read them (of
+ * up to 1024 rows at a time) besides the counters and partial tiles, and need not be zero-filled. */
 #define FK_SCHEDULE_TILES 3
 /* FK_SCHEDULE_TILES_DIRECT: the same at 8 to 32 rows with the activations staged by the tiles; the
  * workspace is the counters and partial tiles only (none without K splits), zero-filled as
@@ -156,7 +155,7 @@ int fk_arc_w4a16_plan_for(int batch, int n, int k, int group_size, int activatio
 
 /* Packet GEMV in one launch with fp16 or bf16 activations (FK_ACT_*), output in the same dtype,
  * and a caller-owned workspace: at least plan.workspace_bytes, 256-byte aligned, zero-filled
- * before its first use (every call leaves it zero-filled). Calls sharing a workspace must be
+ * before its first use (every call leaves its first 64 KB, the counters, zero). Calls sharing one must be
  * stream-ordered. Capturable into a HIP graph (no allocation, no memset). */
 int fk_arc_w4a16_forward_ex(const void* activations, const void* packets, void* output,
                             void* workspace, size_t workspace_bytes, int batch, int n, int k,
@@ -219,8 +218,9 @@ int fk_arc_w4a16_forward_native(const void* activations, const void* packets, vo
                                 int group_size, int packet_format, int activation_dtype,
                                 int split_k_slices, void* stream);
 
-/* fk_arc_w4a16_forward_native with the automatic plan, for callers that cannot allocate (code under
- * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the
+/* fk_arc_w4a16_forward_native with no workspace, for callers that cannot allocate (code under
+ * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the automatic plan, except
+ * that it never takes the row tiles (FK_SCHEDULE_TILES*). No counterpart in the
  * reference. It takes no workspace and calls no hipMalloc / hipFree: the stream-K fix-up scratch
  * is a file-scope device array of FK_NOALLOC_SCRATCH_BYTES that every GPU the library runs on
  * holds until the process ends, set up on the first call on a device (address lookup and one
@@ -230,7 +230,8 @@ int fk_arc_w4a16_forward_native(const void* activations, const void* packets, vo
  * ordered on one stream do not. As a guard, a call whose plan uses the scratch fails with
  * FK_ERR_RUNTIME when the previous such call on that GPU came from another stream that still has
  * work queued (not checked while the calling stream is being captured). Results are those of
- * fk_arc_w4a16_forward_native. */
+ * fk_arc_w4a16_forward_native; where that runs the row tiles (from 8 rows), up to the order of the
+ * fp32 sums. Every automatic plan of up to 16 rows and N up to 131072 fits the array. */
 #define FK_NOALLOC_SCRATCH_BYTES (8388608 + 65536)
 int fk_w4a16_forward_noalloc(const void* activations, const void* packets, void* output, int batch,
                              int n, int k, int group_size, int packet_format,

@@ -1,6 +1,6 @@
 """fk_w4a16_forward_noalloc (the entry point that allocates nothing) through the C ABI, against
-fk_arc_w4a16_forward_native with a caller workspace: the same plan and kernels, so the outputs
-must be identical bit for bit. Two calls in a row, the second with a smaller input, both on
+fk_arc_w4a16_forward_native with a caller workspace, at rows and shapes whose automatic plan is not the
+row tiles': the same plan and kernels, so the outputs must be identical bit for bit. Two calls in a row, the second with a smaller input, both on
 shapes whose plans split slices across workgroups (so the fixed scratch array carries the
 fix-up counters and partials), and again in reverse size order."""
 
