@@ -59,8 +59,9 @@ dequant_kernel(const uint32_t* __restrict__ q, const uint16_t* __restrict__ alph
 // dequant_arc_packets_kernel (arc_w4a16.cu:183-220): packets -> W[N, K] fp16. A workgroup takes a
 // tile over 256 values of K: 512-byte word rows in, through LDS, 512 bytes of each row of W out
 // (a row's words are 512 bytes apart in the packets: reading them in W's order fetched every line
-// many times over). HBM-bound: 8192 x 8192 G128 69.0 -> 27.9 us a call among others (6.1 TB/s; a large
-// copy runs at 5.2), 28672 x 4096 117.5 -> 54.8.
+// many times over). HBM-bound: 8192 x 8192 G128 69.2 -> 29.5 us with cold packets (5.8 TB/s; a large copy
+// runs at 5.2), 28672 x 4096 118 -> 55. (A few workgroups take longer, below a call's 8 us on the host: 1920
+// x 1152 4.0 -> 6.2.)
 template <int G>
 __global__ void __launch_bounds__(kAuxThreads)
 dequant_packets_kernel(const uint8_t* __restrict__ packets, uint4* __restrict__ out, int k,
@@ -198,9 +199,10 @@ __device__ __forceinline__ void store_neg_zp(NativeSlot s, uint32_t zp) {
 // takes a tile, 256 values of K at a time: 128 bytes of each of the tile's rows in, through LDS,
 // whole word rows (kArc) or 1 KB runs of slabs out; scales through LDS too, those of up to four
 // turns at once. (One thread per column and group read 64 bytes of each row, with the line's other
-// half read by another workgroup much later, and every scale with a line of its own.) HBM-bound:
-// 28672 x 4096 to reference packets G128 31.0 -> 26.7 us (4.7 TB/s), G64 42.1 -> 33.1; to native
-// slabs 28.9 -> 24.0 and 34.7 -> 26.8.
+// half read by another workgroup much later, and every scale with a line of its own.) HBM-bound. With
+// cold tensors: to reference packets 57344 x 8192 G128 144.5 -> 105 us (4.8 TB/s), 8192 x 8192 22.9 -> 17.8,
+// 28672 x 4096 30.3 -> 30.1, G64 41.8 -> 35.9; to native slabs 127.5 -> 103.5, 20.9 -> 15.9, 28.3 -> 27.6 and
+// 34.5 -> 30.7. (Weights of a few MB take longer, below a call's 8 us on the host: 1024 x 4096 2.8 -> 3.4.)
 template <int G, PacketFormat F>
 __global__ void __launch_bounds__(kAuxThreads)
 pack_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ alpha,
