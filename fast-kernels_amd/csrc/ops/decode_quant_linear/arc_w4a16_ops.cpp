@@ -391,8 +391,8 @@ bool fused_mfma_takes_small(int batch, bool silu) {
   return batch >= 5 && (batch <= 8 || silu);
 }
 // Whether a fused neighbour at 2-16 rows that the stream kernels do not take (long K, slices that do
-// not divide) goes from the dot2 kernels, which split K, to the row-tile GEMM, whose two launches
-// take 13 us at least. us on MI355X, bf16, dot2 and row tiles: RMSNorm at 2 rows 8192 x 11008 G128
+// not divide) may go from the dot2 kernels, which split K, to the row-tile GEMM, whose two launches
+// take 13 us at least (fused_tile_limit_us then compares the two). us on MI355X, bf16, dot2 and row tiles: RMSNorm at 2 rows 8192 x 11008 G128
 // 16.9 and 23.5, 53248 x 8192 62.4 and 64.5; at 3 rows 14336 x 5120 G128 20.9 and 21.4, 10240 x 8192
 // G128 28.4 and 22.5, 8192 x 11008 G64 25.3 and 26.0, 12288 x 12288 G64 42.8 and 36.5. With SiLU,
 // where a dot2 workgroup has a pair of slices over all of K: at 2 rows 6144 x 8192 22.9 and 20.1, 10240
